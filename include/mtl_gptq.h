@@ -332,6 +332,24 @@ int mtl_w4_gemm_prefill_qsz(const void* x, int64_t M, int64_t ldx, int64_t K,
                             int64_t ldy, float* workspace, int64_t ws_bytes, void* stream);
 
 /*
+ * The same product for prompts of many rows, with the weights dequantised on the way to the
+ * matrix cores and x rescaled per row, both exact in f16 (csrc/mtl_w4wide.hip): two launches,
+ * x [M, ldx] and the metadata into `workspace`, then the GEMM with the same epilogues and
+ * output types.  K % 256 == 0 (<= 65536), N % 16 == 0 (SiLU*up: N % 64 == 0), rows of x
+ * 16-byte aligned; any M up to 2^20.
+ * The size query returns the workspace's bytes where this GEMM is the faster one and 0 where
+ * mtl_w4_gemm_prefill_qsz is; the call itself runs at any M, given 16-byte aligned workspace of
+ * ceil(M/16) (K/32 + 3 G) 1024 + (N/16) G 1024 + (K/g) N 2 + 16 + 64 ceil(M/16) + 4 N bytes,
+ * G = ceil(K/g/32) (MTL_ERR_WORKSPACE if it is smaller).
+ */
+int64_t mtl_w4_gemm_prompt_qsz_workspace_bytes(int64_t M, int64_t K, int64_t N,
+                                               int32_t group_size);
+int mtl_w4_gemm_prompt_qsz(const void* x, int64_t M, int64_t ldx, int64_t K,
+                           const int32_t* strip_weight, const void* qsz, int64_t N,
+                           int32_t group_size, int32_t epilogue, int32_t out_dtype, void* y,
+                           int64_t ldy, void* workspace, int64_t ws_bytes, void* stream);
+
+/*
  * The prompt-length GEMM's K-split partial sums only, for a caller that adds the splits
  * itself (mtl_qk_norm_rope_kv_rows_partials, mtl_residual_rmsnorm_gather: the split sum
  * and the next operation in one launch instead of the second launch and that one).

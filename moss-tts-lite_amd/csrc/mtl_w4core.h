@@ -205,6 +205,17 @@ int strip_rows(const void* x, int64_t M, int64_t ldx, int64_t K, const int32_t* 
                int32_t group_size, int32_t zero_offset, int fmt, void* y, int64_t ldy,
                int32_t out_dtype, void* stream);
 
+// The prompt-length GEMM on the reference's records with dequantised f16 operands
+// (mtl_w4wide.hip): whether it is the faster one for a shape (group 0: at any group size), the
+// workspace it needs (largest at group 32), and its launches.  Pointers, alignment and the
+// K % 256, N % 16 and K % group rules are checked by the caller.
+int pf_device_cus();
+bool wide_pays(int64_t M, int64_t K, int64_t N, int32_t group);
+int64_t wide_workspace_bytes(int64_t M, int64_t K, int64_t N, int32_t group);
+int wide_gemm(const void* x, int64_t M, int64_t ldx, int64_t K, const int32_t* strip_weight,
+              const void* qsz, int64_t N, int32_t group, int32_t epilogue, bool out_f32, void* y,
+              int64_t ldy, void* workspace, hipStream_t st);
+
 // Whether the skinny-batch strip GEMM pays at M rows over N columns (without an act-order
 // gather): measured on MI355X it is ahead of the prompt-length GEMM at every M <= 16 on the
 // four decode shapes, g32 and g128 (q|k|v 6.5-9.1 against 14.2-17.7 us, down 9.8-21.9

@@ -427,7 +427,7 @@ static int prefill_splits(int64_t tiles, int64_t kb, int cus) {
 
 static int g_pf_cus = 0;
 
-static int pf_device_cus() {
+int pf_device_cus() {
   if (!g_pf_cus) {
     int dev = 0, n = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -666,12 +666,16 @@ static bool int4pack_prefill(int64_t M, int64_t N) {
 }
 
 int64_t mtl_int4pack_mm_workspace_bytes(int64_t M, int64_t K, int64_t N) {
-  return M > 1 && int4pack_prefill(M, N) ? mtl_w4_gemm_prefill_workspace_bytes(M, K, N) : 0;
+  const int64_t split =
+      M > 1 && int4pack_prefill(M, N) ? mtl_w4_gemm_prefill_workspace_bytes(M, K, N) : 0;
+  const int64_t wide = wide_pays(M, K, N, 0) ? wide_workspace_bytes(M, K, N, 32) : 0;
+  return split > wide ? split : wide;
 }
 
 // The drop-in for torch._weight_int4pack_mm: M = 1 on the full-K strip GEMV, 2 to 16 rows on
-// the skinny strip GEMM (strip_rows_pays), more on the prompt-length GEMM (or, when N is not
-// a multiple of 128, the skinny GEMM 16 rows at a time).
+// the skinny strip GEMM (strip_rows_pays), more on the GEMM with dequantised operands where
+// it pays (wide_pays) and the workspace holds its operands, else on the prompt-length GEMM
+// (or, when N is not a multiple of 128, the skinny GEMM 16 rows at a time).
 int mtl_int4pack_mm(const void* x, int64_t M, int64_t K, const int32_t* packed,
                     int32_t group_size, const void* qsz, int64_t N, void* y, void* workspace,
                     int64_t ws_bytes, void* stream) {
@@ -699,6 +703,10 @@ int mtl_int4pack_mm(const void* x, int64_t M, int64_t K, const int32_t* packed,
     sa.y16 = static_cast<uint16_t*>(y);
     return strip_launch(sa, st);
   }
+  if (wide_pays(M, K, N, group_size) && workspace && aligned16(workspace) &&
+      ws_bytes >= wide_workspace_bytes(M, K, N, group_size))
+    return wide_gemm(x, M, K, K, packed, qsz, N, group_size, MTL_EPI_NONE, false, y, N, workspace,
+                     st);
   if (int4pack_prefill(M, N))
     return prefill_gemm(x, M, K, K, packed, qsz, nullptr, N, group_size, 0, MTL_EPI_NONE,
                         MTL_OUT_BF16, y, N, static_cast<float*>(workspace), ws_bytes,

@@ -684,6 +684,41 @@ class FastDecoder:
         self._pf = pf
         return pf
 
+    def _wide_bytes(self, rows: int, lin) -> int:
+        """Workspace bytes of the dequantised-operand GEMM where ``lin`` runs ``rows`` prompt
+        rows on it (mtl_w4_gemm_prompt_qsz: plain x in, no split partials), else 0."""
+        if lin.stream_weight(True)[1] != N.LAYOUT_STRIP_QSZ:
+            return 0
+        return int(N.load().mtl_w4_gemm_prompt_qsz_workspace_bytes(
+            rows, lin.in_features, lin.out_features, lin.group_size))
+
+    def _prefill_wide(self, x, rows: int, lin, epilogue: int, y, ldy: int, stream) -> None:
+        """One prompt-length GEMM of the reference's records on plain x
+        (mtl_w4_gemm_prompt_qsz), its operands staged in this decoder's own buffer."""
+        pf = self._pf
+        nbytes = self._wide_bytes(rows, lin)
+        if pf.get("wide") is None or pf["wide"].numel() < nbytes:
+            pf["wide"] = torch.empty(nbytes, dtype=torch.uint8, device=self.dev)
+        N.check(N.load().mtl_w4_gemm_prompt_qsz(
+            x.data_ptr(), rows, x.stride(0), lin.in_features, lin.packed.data_ptr(),
+            lin.qsz.data_ptr(), lin.out_features, lin.group_size, epilogue, N.OUT_BF16,
+            y.data_ptr(), ldy, pf["wide"].data_ptr(), pf["wide"].numel(), stream),
+            "mtl_w4_gemm_prompt_qsz")
+
+    def _prefill_norm(self, rows: int, norm_w, nxt, out, stream) -> None:
+        """``out = RMSNorm(h)`` in the input order of ``nxt``, staged for its GEMM when that
+        takes staged x."""
+        cfg, pf, lib = self.m.cfg, self._pf, N.load()
+        args = (pf["h"].data_ptr(), cfg.hidden, norm_w.data_ptr(),
+                None if nxt.perm is None else nxt.perm.data_ptr(), out.data_ptr(), cfg.hidden)
+        if self._prefill_staged() and not self._wide_bytes(rows, nxt):
+            N.check(lib.mtl_rmsnorm_gather_staged(*args, pf["xsum"].data_ptr(), rows, cfg.hidden,
+                                                  ctypes.c_float(cfg.eps), stream),
+                    "mtl_rmsnorm_gather_staged")
+        else:
+            N.check(lib.mtl_rmsnorm_gather(*args, rows, cfg.hidden, ctypes.c_float(cfg.eps),
+                                           stream), "mtl_rmsnorm_gather")
+
     def _prefill_gemm(self, x, rows: int, lin, epilogue: int, y, ldy: int, stream) -> None:
         """One prompt-length int4 GEMM on the strip copy of ``lin`` (mtl_w4_gemm_prefill,
         or mtl_w4_gemm_prefill_qsz for the reference's records)."""
@@ -741,26 +776,28 @@ class FastDecoder:
             "mtl_w4_gemm_prefill_partials")
         return int(lib.mtl_w4_gemm_prefill_partials_bytes(rows, K, Nc)) // (rows * Nc * 4)
 
-    def _prefill_residual_norm(self, x_in, rows: int, lin, norm_w, gather, out, stream) -> None:
-        """``h += x_in @ lin`` and ``out = RMSNorm(h)`` gathered by ``gather``: the GEMM's
-        split partials, then the split sum, residual add and norm in one launch (the bits
-        of the GEMM's residual launch followed by mtl_rmsnorm_gather), out staged for the
-        next GEMM when the prompt stages x."""
+    def _prefill_residual_norm(self, x_in, rows: int, lin, norm_w, nxt, out, stream) -> None:
+        """``h += x_in @ lin`` and ``out = RMSNorm(h)`` in the input order of ``nxt``: the
+        GEMM's split partials, then the split sum, residual add and norm in one launch (the
+        bits of the GEMM's residual launch followed by mtl_rmsnorm_gather), out staged for
+        ``nxt`` when its GEMM takes staged x.  A GEMM without split partials adds into h
+        itself and the norm follows."""
         cfg, pf = self.m.cfg, self._pf
         h, part = pf["h"], pf["part"]
-        if not self.fuse_split_sums:
-            self._prefill_gemm(x_in, rows, lin, N.EPI_RESIDUAL, h, cfg.hidden, stream)
-            N.check(N.load().mtl_rmsnorm_gather(
-                h.data_ptr(), cfg.hidden, norm_w.data_ptr(),
-                None if gather is None else gather.data_ptr(), out.data_ptr(), cfg.hidden,
-                rows, cfg.hidden, ctypes.c_float(cfg.eps), stream), "mtl_rmsnorm_gather")
+        wide = self._wide_bytes(rows, lin)
+        if wide or not self.fuse_split_sums:
+            gemm = self._prefill_wide if wide else self._prefill_gemm
+            gemm(x_in, rows, lin, N.EPI_RESIDUAL, h, cfg.hidden, stream)
+            self._prefill_norm(rows, norm_w, nxt, out, stream)
             return
+        gather = nxt.perm
+        staged = self._prefill_staged() and not self._wide_bytes(rows, nxt)
         splits = self._prefill_partials(x_in, rows, lin, part, stream)
         N.check(N.load().mtl_residual_rmsnorm_gather(
             part.data_ptr(), splits, part.numel() * 4, h.data_ptr(), cfg.hidden,
             norm_w.data_ptr(),
             None if gather is None else gather.data_ptr(), out.data_ptr(), cfg.hidden,
-            pf["xsum"].data_ptr() if self._prefill_staged() else None, rows, cfg.hidden,
+            pf["xsum"].data_ptr() if staged else None, rows, cfg.hidden,
             ctypes.c_float(cfg.eps), stream), "mtl_residual_rmsnorm_gather")
 
     def prefill_rows(self, ids: torch.Tensor, pos0: int = 0) -> torch.Tensor:
@@ -788,33 +825,31 @@ class FastDecoder:
                                    self.table_ptrs.data_ptr(), self.vocabs.data_ptr(), cfg.hidden,
                                    h.data_ptr(), st), "mtl_embed_rows")
         n_layers = len(m.layers)
-        staged = self._prefill_staged()
-        xsum = pf["xsum"] if staged else None
         for li, lyr in enumerate(m.layers):
             lq = lyr["qkv"]
-            if li == 0 and staged:   # later layers' input norms ride on the previous down GEMM
-                N.check(lib.mtl_rmsnorm_gather_staged(
-                    h.data_ptr(), cfg.hidden, lyr["input_layernorm"].data_ptr(), p(lq.perm),
-                    x.data_ptr(), cfg.hidden, xsum.data_ptr(), rows, cfg.hidden, eps, st),
-                    "mtl_rmsnorm_gather_staged")
-            elif li == 0:
-                N.check(lib.mtl_rmsnorm_gather(h.data_ptr(), cfg.hidden,
-                                               lyr["input_layernorm"].data_ptr(),
-                                               p(lq.perm), x.data_ptr(), cfg.hidden, rows,
-                                               cfg.hidden, eps, st), "mtl_rmsnorm_gather")
-            fuse_qkv = self.fuse_split_sums
-            if fuse_qkv:
-                splits = self._prefill_partials(x, rows, lq, pf["part"], st, xsum)
+            if li == 0:   # later layers' input norms ride on the previous down GEMM
+                self._prefill_norm(rows, lyr["input_layernorm"], lq, x, st)
+            wide = self._wide_bytes(rows, lq)
+            staged = self._prefill_staged() and not wide
+            fuse_qkv = self.fuse_split_sums and not wide
+            if wide:
+                self._prefill_wide(x, rows, lq, N.EPI_NONE, qkv, cfg.qkv_out, st)
+            elif fuse_qkv:
+                splits = self._prefill_partials(x, rows, lq, pf["part"], st,
+                                                pf["xsum"] if staged else None)
             else:
                 self._prefill_gemm(x, rows, lq, N.EPI_NONE, qkv, cfg.qkv_out, st)
             if self.v_keep[li]:
                 # the bf16-kept v_proj (gptq.py:689-693) reads x in its natural order
-                N.check(lib.mtl_rmsnorm_gather(h.data_ptr(), cfg.hidden,
-                                               lyr["input_layernorm"].data_ptr(), None,
-                                               pf["x_nat"].data_ptr(), cfg.hidden, rows,
-                                               cfg.hidden, eps, st), "mtl_rmsnorm_gather")
+                x_v = x
+                if lq.perm is not None or staged:
+                    x_v = pf["x_nat"]
+                    N.check(lib.mtl_rmsnorm_gather(h.data_ptr(), cfg.hidden,
+                                                   lyr["input_layernorm"].data_ptr(), None,
+                                                   x_v.data_ptr(), cfg.hidden, rows,
+                                                   cfg.hidden, eps, st), "mtl_rmsnorm_gather")
                 qkv[:rows, lq.out_features:] = torch.nn.functional.linear(
-                    pf["x_nat"][:rows], lyr["v_keep"])
+                    x_v[:rows], lyr["v_keep"])
             if fuse_qkv:   # the split sum rides on the q/k norm launch
                 part = pf["part"]
                 N.check(lib.mtl_qk_norm_rope_kv_rows_partials(
@@ -835,12 +870,18 @@ class FastDecoder:
                 attn.data_ptr(), cfg.hidden, p(self.inv_perm_o[li]), H, Hkv, D, cfg.max_seq,
                 scale, st), "mtl_prefill_attention")
             self._prefill_residual_norm(attn, rows, lyr["o"], lyr["post_attention_layernorm"],
-                                        lyr["gate_up"].perm, x, st)
+                                        lyr["gate_up"], x, st)
+            wide = self._wide_bytes(rows, lyr["gate_up"])
+            staged = self._prefill_staged() and not wide
+            xsum = pf["xsum"] if staged else None
             if self.up_keep[li]:
                 # int4 gate and the bf16-kept up_proj (gptq.py:689-693), then SiLU(gate) * up
                 # in bf16 as the reference's MLP forms it (model.py:40-44)
                 gate = pf["gate"]
-                if staged:
+                if wide:
+                    self._prefill_wide(x, rows, lyr["gate_up"], N.EPI_NONE, gate,
+                                       cfg.intermediate, st)
+                elif staged:
                     self._prefill_gemm_staged(x, xsum, rows, lyr["gate_up"], N.EPI_NONE, gate,
                                               cfg.intermediate, st)
                 else:
@@ -855,6 +896,9 @@ class FastDecoder:
                                                    cfg.hidden, eps, st), "mtl_rmsnorm_gather")
                 up = torch.nn.functional.linear(x_up[:rows], lyr["up_keep"])
                 torch.mul(torch.nn.functional.silu(gate[:rows]), up, out=act[:rows])
+            elif wide:
+                self._prefill_wide(x, rows, lyr["gate_up"], N.EPI_SILU_MUL, act,
+                                   cfg.intermediate, st)
             elif staged:
                 self._prefill_gemm_staged(x, xsum, rows, lyr["gate_up"], N.EPI_SILU_MUL, act,
                                           cfg.intermediate, st)
@@ -864,9 +908,11 @@ class FastDecoder:
             if li + 1 < n_layers:   # the residual add and the next layer's input norm
                 nxt = m.layers[li + 1]
                 self._prefill_residual_norm(act, rows, lyr["down"], nxt["input_layernorm"],
-                                            nxt["qkv"].perm, x, st)
+                                            nxt["qkv"], x, st)
             else:
-                self._prefill_gemm(act, rows, lyr["down"], N.EPI_RESIDUAL, h, cfg.hidden, st)
+                gemm = self._prefill_wide if self._wide_bytes(rows, lyr["down"]) else \
+                    self._prefill_gemm
+                gemm(act, rows, lyr["down"], N.EPI_RESIDUAL, h, cfg.hidden, st)
         return h[:rows]
 
     def _final_norm_row(self, h_row: torch.Tensor) -> None:

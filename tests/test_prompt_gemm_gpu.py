@@ -1,0 +1,140 @@
+"""GPU parity of the GEMM with dequantised operands on the reference's records
+(``mtl_w4_gemm_prompt_qsz``) against float64, and the routes that take it.
+
+fp32 output: the products are exact and the sums run in float32 over K, so the relative error
+is a few times 2^-24 sqrt(K / 32) at most, with a margin 2e-6 at K <= 4608; bf16 output adds
+its rounding, 2^-9 / sqrt(3) of each value (relative 2-norm 1.7e-3, bar 2.5e-3).
+"""
+import pytest
+import torch
+
+from moss_tts_lite_amd import _native as N
+from moss_tts_lite_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def record(dev, n, k, g, seed, s_exp=0):
+    gen = torch.Generator(device=dev).manual_seed(seed)
+    q = torch.randint(0, 16, (n, k), device=dev, generator=gen)
+    pre = (q[:, 1::2] | (q[:, 0::2] << 4)).to(torch.uint8)
+    s = torch.rand(k // g, n, device=dev, generator=gen) * 0.004 + 0.002
+    z = torch.randn(k // g, n, device=dev, generator=gen) * 0.002
+    qsz = (torch.stack([s, z], -1) * 2.0 ** s_exp).bfloat16()
+    sc, zr = (qsz[..., i].t().double().repeat_interleave(g, 1) for i in (0, 1))
+    return ops.convert_weight_to_int4pack(pre.contiguous(), 8), qsz, (q.double() - 8) * sc + zr
+
+
+def workspace(m, k, n, g, dev):
+    t, c = (m + 15) // 16, -(-(k // g) // 32)
+    return torch.empty(t * (k // 32 + 3 * c) * 1024 + n // 16 * c * 1024 + k // g * n * 2 + 16
+                       + 64 * t + 4 * n, dtype=torch.uint8, device=dev)
+
+
+def run(x, packed, qsz, g, epilogue, y, ldx=None):
+    m, k = x.shape
+    n = qsz.shape[1]
+    ws = workspace(m, k, n, g, x.device)
+    N.check(N.load().mtl_w4_gemm_prompt_qsz(
+        x.data_ptr(), m, x.stride(0), k, packed.data_ptr(), qsz.data_ptr(), n, g, epilogue,
+        N.OUT_F32 if y.dtype == torch.float32 else N.OUT_BF16, y.data_ptr(), y.stride(0),
+        ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream), "prompt gemm")
+    torch.cuda.synchronize()
+    return y
+
+
+def rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+# every count of row tiles per workgroup (1 .. 6), a ragged last tile, ragged column tiles, one
+# and several turns (K = 256: one block per wave group; 1792: 7 blocks), every group size
+@pytest.mark.parametrize("m,k,n,g", [
+    (1, 256, 16, 32), (16, 512, 256, 256), (17, 768, 272, 128), (33, 1792, 336, 64),
+    (65, 1024, 1040, 32), (97, 4608, 256, 256), (389, 1024, 4096, 32), (600, 512, 5120, 128),
+    (1100, 768, 4096, 64), (1536, 512, 4096, 128),
+])
+def test_prompt_gemm_matches_float64(dev, m, k, n, g):
+    packed, qsz, w = record(dev, n, k, g, m + k + n)
+    gen = torch.Generator(device=dev).manual_seed(7)
+    xb = torch.randn(m, k + 8, device=dev, generator=gen)
+    xb[:, ::37] *= 50.0
+    x = xb.bfloat16()[:, :k]                     # a row pitch of its own
+    ref = x.double() @ w.t()
+    y = run(x, packed, qsz, g, N.EPI_NONE, torch.empty(m, n, device=dev))
+    assert rel(y, ref) < 2e-6
+    # rows 4 bytes off a 16-byte pitch: the unpacked stores
+    wide = torch.zeros(m, n + 1, device=dev)
+    assert torch.equal(run(x, packed, qsz, g, N.EPI_NONE, wide[:, :n]), y) and not wide[:, n:].any()
+    yb = run(x, packed, qsz, g, N.EPI_NONE, torch.empty(m, n, device=dev, dtype=torch.bfloat16))
+    assert torch.equal(yb, y.bfloat16())
+    h = torch.randn(m, n, device=dev, generator=gen).bfloat16()
+    hr = (y.bfloat16().float() + h.float()).bfloat16()
+    assert torch.equal(run(x, packed, qsz, g, N.EPI_RESIDUAL, h), hr)
+    if n % 64 == 0:
+        act = run(x, packed, qsz, g, N.EPI_SILU_MUL,
+                  torch.empty(m, n // 2, device=dev, dtype=torch.bfloat16))
+        gu = y.bfloat16().float().reshape(m, n // 64, 2, 32)
+        want = torch.nn.functional.silu(gu[:, :, 0]).bfloat16().float() * gu[:, :, 1]
+        # the hardware exp and reciprocal: one bf16 ulp where the quotient is near a boundary
+        assert rel(act, want.reshape(m, -1).double()) < 2.5e-3
+
+
+def test_prompt_gemm_ranges(dev):
+    # scales and activations far from 1, an all-zero row and an all-zero column: the powers of
+    # two found per row and column keep the operands in f16's range; a row with an infinity is
+    # not finite and leaves the others alone
+    m, k, n, g = 70, 1024, 512, 64
+    gen = torch.Generator(device=dev).manual_seed(3)
+    base = torch.randn(m, k, device=dev, generator=gen)
+    for x_exp, s_exp in ((0, 0), (60, -60), (-70, 40), (30, 10), (-40, -40)):
+        packed, qsz, w = record(dev, n, k, g, 5, s_exp)
+        qsz[:, 3] = 0
+        w[3] = 0
+        x = (base * 2.0 ** x_exp).bfloat16()
+        x[11] = 0
+        y = run(x, packed, qsz, g, N.EPI_NONE, torch.empty(m, n, device=dev))
+        ref = x.double() @ w.t()
+        assert rel(y, ref) < 2e-6 and not y[11].any() and not y[:, 3].any()
+        xi = x.clone()
+        xi[5, 100] = float("inf")
+        yi = run(xi, packed, qsz, g, N.EPI_NONE, torch.empty(m, n, device=dev))
+        keep = torch.arange(m, device=dev) != 5
+        assert torch.equal(yi[keep], y[keep]) and not torch.isfinite(yi[5, :3]).any()
+
+
+def test_prompt_gemm_checks(dev):
+    packed, qsz, _ = record(dev, 256, 512, 32, 1)
+    x = torch.zeros(20, 512, device=dev, dtype=torch.bfloat16)
+    y = torch.empty(20, 256, device=dev, dtype=torch.bfloat16)
+    ws = workspace(20, 512, 256, 32, dev)
+
+    def call(m=20, k=512, n=256, g=32, epi=0, wsn=ws.numel(), ldy=256):
+        return N.load().mtl_w4_gemm_prompt_qsz(
+            x.data_ptr(), m, 512, k, packed.data_ptr(), qsz.data_ptr(), n, g, epi, N.OUT_BF16,
+            y.data_ptr(), ldy, ws.data_ptr(), wsn, torch.cuda.current_stream().cuda_stream)
+
+    assert call() == 0
+    torch.cuda.synchronize()
+    for bad in (dict(m=0), dict(k=384), dict(n=248), dict(g=48), dict(epi=9), dict(ldy=128),
+                dict(wsn=ws.numel() - 64)):
+        assert call(**bad) < 0, bad
+
+
+@pytest.mark.parametrize("m,k,n,g", [(300, 1024, 2000, 32), (389, 4096, 24576, 32), (700, 4096, 6144, 64)])
+def test_int4pack_mm_route(dev, m, k, n, g):
+    # the drop-in takes this GEMM for many rows: the same bits, also replayed from a graph
+    assert N.load().mtl_w4_gemm_prompt_qsz_workspace_bytes(m, k, n, g) > 0
+    packed, qsz, w = record(dev, n, k, g, 9)
+    x = torch.randn(m, k, device=dev).bfloat16()
+    y = ops.weight_int4pack_mm(x, packed, g, qsz)
+    want = run(x, packed, qsz, g, N.EPI_NONE, torch.empty_like(y))
+    assert torch.equal(y, want) and rel(y, x.double() @ w.t()) < 2.5e-3
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops.weight_int4pack_mm(x, packed, g, qsz)
+    for i in range(3):
+        x.copy_(torch.randn(m, k, device=dev).bfloat16())
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ops.weight_int4pack_mm(x, packed, g, qsz)), i
