@@ -5,6 +5,8 @@ fp32 output: the products are exact and the sums run in float32 over K, so the r
 is a few times 2^-24 sqrt(K / 32) at most, with a margin 2e-6 at K <= 4608; bf16 output adds
 its rounding, 2^-9 / sqrt(3) of each value (relative 2-norm 1.7e-3, bar 2.5e-3).
 """
+import ctypes
+
 import pytest
 import torch
 
@@ -138,3 +140,25 @@ def test_int4pack_mm_route(dev, m, k, n, g):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, ops.weight_int4pack_mm(x, packed, g, qsz)), i
+
+
+def test_embed_rows_unaligned_table(dev):
+    # 11 tables (more than one set of 8), one of them 2 bytes off a 16-byte boundary
+    hidden, rows = 72, 5
+    gen = torch.Generator(device=dev).manual_seed(2)
+    store = [torch.randn(30 * hidden + 1, device=dev, generator=gen).bfloat16() for _ in range(11)]
+    tabs = [t[(1 if i == 4 else 0):][:30 * hidden].reshape(30, hidden) for i, t in enumerate(store)]
+    ids = torch.randint(-1, 31, (rows, 11), device=dev, generator=gen)
+    ptrs = torch.tensor([t.data_ptr() for t in tabs], dtype=torch.int64, device=dev)
+    vocabs = torch.full((11,), 30, dtype=torch.int64, device=dev)
+    out = torch.empty(rows, hidden, dtype=torch.bfloat16, device=dev)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    N.check(N.load().mtl_embed_rows(ids.data_ptr(), rows, 11, ptrs.data_ptr(), vocabs.data_ptr(),
+                                    hidden, out.data_ptr(), st), "embed rows")
+    torch.cuda.synchronize()
+    for r in range(rows):
+        h = None
+        for t, i in zip(tabs, ids[r].tolist()):
+            v = t[i] if 0 <= i < 30 else torch.zeros_like(t[0])
+            h = v if h is None else h + v
+        assert torch.equal(out[r], h)
