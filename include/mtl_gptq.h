@@ -350,6 +350,20 @@ int mtl_w4_gemm_prompt_qsz(const void* x, int64_t M, int64_t ldx, int64_t K,
                            int64_t ldy, void* workspace, int64_t ws_bytes, void* stream);
 
 /*
+ * mtl_w4_gemm_prefill on x gathered through the act-order index (row k of the weight is
+ * channel perm[k] of x): one launch gathers and stages x into `workspace`, then the GEMM (the
+ * bits of mtl_w4_gemm_prefill on the gathered x).  perm int32 [K] 16-byte aligned with values
+ * in 0 .. K-1, K <= 16384; the size query returns 0 for shapes it does not take.
+ */
+int64_t mtl_w4_gemm_prefill_gather_workspace_bytes(int64_t M, int64_t K, int64_t N);
+int mtl_w4_gemm_prefill_gather(const void* x, int64_t M, int64_t ldx, int64_t K,
+                               const int32_t* perm, const int32_t* strip_weight,
+                               const void* strip_scales, const int32_t* strip_zeros, int64_t N,
+                               int32_t group_size, int32_t zero_offset, int32_t out_dtype,
+                               void* y, int64_t ldy, void* workspace, int64_t ws_bytes,
+                               void* stream);
+
+/*
  * The prompt-length GEMM's K-split partial sums only, for a caller that adds the splits
  * itself (mtl_qk_norm_rope_kv_rows_partials, mtl_residual_rmsnorm_gather: the split sum
  * and the next operation in one launch instead of the second launch and that one).

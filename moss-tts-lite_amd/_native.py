@@ -128,6 +128,10 @@ _SIGNATURES = {
     "mtl_w4_gemm_prefill_qsz": (_i32, [_c_void_p, _i64, _i64, _i64, _c_void_p, _c_void_p, _i64,
                                        _i32, _i32, _i32, _c_void_p, _i64, _c_void_p, _i64,
                                        _c_void_p]),
+    "mtl_w4_gemm_prefill_gather_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "mtl_w4_gemm_prefill_gather": (_i32, [_c_void_p, _i64, _i64, _i64, _c_void_p, _c_void_p,
+                                          _c_void_p, _c_void_p, _i64, _i32, _i32, _i32, _c_void_p,
+                                          _i64, _c_void_p, _i64, _c_void_p]),
     "mtl_w4_gemm_prompt_qsz_workspace_bytes": (_i64, [_i64, _i64, _i64, _i32]),
     "mtl_w4_gemm_prompt_qsz": (_i32, [_c_void_p, _i64, _i64, _i64, _c_void_p, _c_void_p, _i64,
                                       _i32, _i32, _i32, _c_void_p, _i64, _c_void_p, _i64,

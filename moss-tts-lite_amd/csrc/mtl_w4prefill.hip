@@ -582,6 +582,40 @@ static int prefill_gemm(const void* x, int64_t M, int64_t ldx, int64_t K,
   return launch_status();
 }
 
+// x gathered through the act-order index and staged for the GEMM (PRE): a workgroup per row,
+// the row read once, coalesced, into LDS, from which the 2-byte gather runs; each output item
+// in pair order with its 32-channel sums, as rmsnorm_gather_kernel stages them.  Bound by
+// latency: 200 x 4096 in about 5 us (1.6 MB in and out).
+constexpr int kGatherMaxK = 16384;               // 32 KB of LDS
+
+__global__ void __launch_bounds__(256) prefill_gather_kernel(const uint16_t* __restrict__ x,
+                                                             int64_t ldx,
+                                                             const int32_t* __restrict__ perm,
+                                                             u32x4* __restrict__ out,
+                                                             float* __restrict__ sums, int K) {
+  __shared__ u32x4 row4[kGatherMaxK / 8];
+  const u32x4* xr = reinterpret_cast<const u32x4*>(x + (size_t)blockIdx.x * ldx);
+  const int t = threadIdx.x, items = K >> 3;     // a multiple of 32
+  for (int i = t; i < items; i += 256) row4[i] = xr[i];
+  __syncthreads();
+  const uint16_t* row = reinterpret_cast<const uint16_t*>(row4);
+  for (int i0 = 0; i0 < items; i0 += 256) {
+    const int i = i0 + t;
+    const bool in = i < items;                   // whole 32-channel groups are in or out
+    const int4* pp = reinterpret_cast<const int4*>(perm) + 2 * (in ? i : 0);
+    const int4 a = pp[0], b = pp[1];
+    const u32x4 v{row[a.x] | (uint32_t)row[a.y] << 16, row[a.z] | (uint32_t)row[a.w] << 16,
+                  row[b.x] | (uint32_t)row[b.y] << 16, row[b.z] | (uint32_t)row[b.w] << 16};
+    float sum;
+    const u32x4 pv = pair_order_dot(v, sum);
+    sum = group_sum_valu<4>(sum);
+    if (in) {
+      out[(size_t)blockIdx.x * items + i] = pv;
+      if ((i & 3) == 0) sums[(size_t)blockIdx.x * (items >> 2) + (i >> 2)] = sum;
+    }
+  }
+}
+
 }  // namespace mtl
 
 using namespace mtl;
@@ -648,6 +682,48 @@ int mtl_w4_gemm_prefill_staged(const void* x, const float* x_sums, int64_t M, in
                       ldy, workspace, ws_bytes,
                       meta_format == MTL_META_QSZ ? STRIP_META_QSZ : STRIP_META_GPTQ,
                       (hipStream_t)stream, x_sums);
+}
+
+int64_t mtl_w4_gemm_prefill_gather_workspace_bytes(int64_t M, int64_t K, int64_t N) {
+  if (M < 1 || K < 256 || K % 256 != 0 || K > kGatherMaxK || N < kPfCols || N % kPfCols != 0 ||
+      M * K * 2 >= ((int64_t)1 << 31) || (N / 16) * (K / 128) * 1024 >= ((int64_t)1 << 31) ||
+      (K / 32) * N * 2 >= ((int64_t)1 << 31))
+    return 0;
+  return M * K * 2 + M * (K / 32) * 4 + mtl_w4_gemm_prefill_workspace_bytes(M, K, N);
+}
+
+int mtl_w4_gemm_prefill_gather(const void* x, int64_t M, int64_t ldx, int64_t K,
+                               const int32_t* perm, const int32_t* strip_weight,
+                               const void* strip_scales, const int32_t* strip_zeros, int64_t N,
+                               int32_t group_size, int32_t zero_offset, int32_t out_dtype,
+                               void* y, int64_t ldy, void* workspace, int64_t ws_bytes,
+                               void* stream) {
+  if (!x || !perm || !strip_zeros) return MTL_ERR_INVALID_ARG;
+  const int64_t need = mtl_w4_gemm_prefill_gather_workspace_bytes(M, K, N);
+  if (need == 0 || ldx < K) return MTL_ERR_SHAPE;
+  if (!aligned16(x) || ldx % 8 != 0 || !aligned16(perm) || !aligned16(strip_zeros))
+    return MTL_ERR_ALIGN;
+  if (!workspace || ws_bytes < need) return MTL_ERR_WORKSPACE;
+  if (!aligned16(workspace)) return MTL_ERR_ALIGN;
+  char* const ws = static_cast<char*>(workspace);
+  float* const sums = reinterpret_cast<float*>(ws + M * K * 2);
+  float* const part = sums + M * (K / 32);
+  // the GEMM's checks first: nothing is launched for a call that it refuses
+  if (!strip_weight || !strip_scales || !y) return MTL_ERR_INVALID_ARG;
+  if (out_dtype != MTL_OUT_BF16 && out_dtype != MTL_OUT_F32) return MTL_ERR_INVALID_ARG;
+  if (group_size != 32 && group_size != 64 && group_size != 128 && group_size != 256)
+    return MTL_ERR_GROUP;
+  if (ldy < N) return MTL_ERR_SHAPE;
+  if (!aligned16(strip_weight) || !aligned16(strip_scales) ||
+      (reinterpret_cast<uintptr_t>(y) & (out_dtype == MTL_OUT_F32 ? 3u : 1u)))
+    return MTL_ERR_ALIGN;
+  hipStream_t st = (hipStream_t)stream;
+  hipLaunchKernelGGL(prefill_gather_kernel, dim3((unsigned)M), dim3(256), 0, st,
+                     static_cast<const uint16_t*>(x), ldx, perm, reinterpret_cast<u32x4*>(ws), sums,
+                     (int)K);
+  return prefill_gemm(ws, M, K, K, strip_weight, strip_scales, strip_zeros, N, group_size,
+                      zero_offset, MTL_EPI_NONE, out_dtype, y, ldy, part,
+                      ws_bytes - (reinterpret_cast<char*>(part) - ws), STRIP_META_GPTQ, st, sums);
 }
 
 int mtl_w4_gemm_prefill_qsz(const void* x, int64_t M, int64_t ldx, int64_t K,

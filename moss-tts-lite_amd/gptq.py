@@ -153,6 +153,25 @@ class GPTQLinear(torch.nn.Module):
             self._strip_meta = ops.strip_meta(self.scales, self.qzeros, self.group_size)
         return self._strip_meta
 
+    def _prompt_ready(self, x: torch.Tensor) -> bool:
+        """Whether the prompt-length GEMM can take this linear's rows: the strip layout and
+        whole 128-column tiles, and the strip copy and its metadata there.  They are built at
+        the first such call (not inside a graph capture, where they would only be filled at
+        replay, nor on a tensor that stands for another in a trace) and waited for, so that any
+        stream may read them."""
+        if self._strip is None or self._strip_meta is None:
+            if not self.supports_strip() or self.out_features % 128 or \
+                    not self.scales.is_cuda or torch.compiler.is_compiling() or \
+                    type(x) not in (torch.Tensor, torch.nn.Parameter) or \
+                    torch.cuda.is_current_stream_capturing():
+                return False
+            strip = self._strip if self._strip is not None else \
+                ops.strip_weights(self.kernel_args()[0])
+            meta = self._strip_meta or ops.strip_meta(self.scales, self.qzeros, self.group_size)
+            torch.cuda.current_stream(self.scales.device).synchronize()
+            self._strip, self._strip_meta = strip, meta
+        return self.out_features % 128 == 0
+
     def drop_original(self) -> None:
         """Free the unsorted ``qweight`` once the sorted copy exists (load-time memory)."""
         if self._perm is not None:
@@ -187,9 +206,11 @@ class GPTQLinear(torch.nn.Module):
     def forward(self, x: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
         """``x[..., K] @ dequant(W)``.  One row runs on the full-K strip GEMV (x gathered
         through the act-order index while staging), few rows on the skinny strip GEMM where
-        it pays (:func:`ops.strip_rows_pays`); both read the strip copy of the weight, built
-        once and kept.  The others run on the split-K GEMM over the AutoGPTQ layout (or,
-        after :meth:`keep_strip_only`, the prompt-length GEMM over the strip copy).  Calls
+        it pays (:func:`ops.strip_rows_pays`), more than 16 on the prompt-length GEMM (x
+        gathered by a launch before it) where N is a multiple of 128; all read the strip copy
+        of the weight, built once and kept.  The others run on the split-K GEMM over the
+        AutoGPTQ layout, 16 rows at a time (4096 x 24576, g128, act-order: 33 us per 16 rows
+        against 30-70 us for 17 to 256 rows on the prompt-length GEMM).  Calls
         go through the ``torch.ops.mtl`` operators (one dispatcher call, torch's stream and
         allocator)."""
         m = x.numel() // self.in_features if self.in_features else 0
@@ -209,15 +230,14 @@ class GPTQLinear(torch.nn.Module):
                                                    self.out_features, self.group_size,
                                                    self.zero_offset, perm, out_dtype)
         if self._strip_only:
-            # the prompt-length GEMM over the strip copy, x's channels taken into the
-            # weight's (group-sorted) row order first
-            x2 = x.reshape(-1, self.in_features)
-            if perm is not None:
-                x2 = x2.index_select(1, perm.long())
+            # the prompt-length GEMM is all that is left: it raises where N % 128 != 0
             sc, qz = self.strip_meta()
-            y = ops.prefill_gemm(x2.contiguous(), self._strip, sc, qz, self.out_features,
-                                 self.group_size, self.zero_offset, out_dtype=out_dtype)
-            return y.reshape(*x.shape[:-1], self.out_features)
+            return ops.torch_ops().prompt_gemm(x, self._strip, sc, qz, self.out_features,
+                                               self.group_size, self.zero_offset, perm, out_dtype)
+        if m > 16 and self._prompt_ready(x):
+            sc, qz = self._strip_meta
+            return ops.torch_ops().prompt_gemm(x, self._strip, sc, qz, self.out_features,
+                                               self.group_size, self.zero_offset, perm, out_dtype)
         qw, qz, sc, perm = self.kernel_args()
         return ops.gptq_gemm(x, qw, qz, sc, self.group_size, perm=perm,
                              zero_offset=self.zero_offset, out_dtype=out_dtype)

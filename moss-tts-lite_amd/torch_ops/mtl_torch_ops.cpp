@@ -264,6 +264,70 @@ at::Tensor strip_gemv(const at::Tensor& x, const at::Tensor& strip_weight,
   return y.view(out_shape(x, n));
 }
 
+// Prompt rows on the prompt-length GEMM (mtl_w4_gemm_prefill, x gathered through perm first
+// for an act-order linear: mtl_w4_gemm_prefill_gather) over the strip copy of an AutoGPTQ
+// linear and its strip-ordered metadata, kPromptRows rows per launch (byte offsets within x
+// stay in 31 bits), the workspace from torch's caching allocator.
+constexpr int64_t kPromptRows = 8192;
+
+at::Tensor prompt_gemm(const at::Tensor& x, const at::Tensor& strip_weight,
+                       const at::Tensor& strip_scales, const at::Tensor& strip_zeros, int64_t n,
+                       int64_t group_size, int64_t zero_offset,
+                       const c10::optional<at::Tensor>& perm, at::ScalarType out_dtype) {
+  const int64_t K = x.size(-1);
+  TORCH_CHECK(strip_weight.scalar_type() == at::kInt && strip_weight.numel() * 8 == n * K,
+              "strip_weight must be the int32 strip copy of a [", K, ", ", n, "] weight");
+  TORCH_CHECK(strip_scales.scalar_type() == at::kHalf && group_size > 0 &&
+                  strip_scales.numel() == n * K / group_size,
+              "strip_scales must be the fp16 strip-ordered scales (mtl_w4_strip_meta)");
+  TORCH_CHECK(strip_zeros.scalar_type() == at::kInt &&
+                  strip_zeros.numel() == n / 8 * (K / group_size),
+              "strip_zeros must be the int32 strip-ordered zeros (mtl_w4_strip_meta)");
+  at::Tensor x2 = rows_of(x, K);
+  TORCH_CHECK(x2.is_cuda() && strip_weight.device() == x2.device() &&
+                  strip_scales.device() == x2.device() && strip_zeros.device() == x2.device(),
+              "x and the strip tensors must be on one HIP device");
+  const c10::DeviceGuard guard(x2.device());
+  // the kernels read x in 16-byte pieces: a view at another offset is copied
+  if (reinterpret_cast<uintptr_t>(x2.data_ptr()) & 15u) x2 = x2.clone();
+  at::Tensor pk;
+  const int32_t* pp = perm_ptr(perm, K, pk);
+  if (pp && (reinterpret_cast<uintptr_t>(pp) & 15u)) {
+    pk = pk.clone();
+    pp = pk.data_ptr<int32_t>();
+  }
+  const at::Tensor w = strip_weight.contiguous(), sc = strip_scales.contiguous(),
+                   z = strip_zeros.contiguous();
+  const int64_t M = x2.size(0);
+  at::Tensor y = at::empty({M, n}, x2.options().dtype(out_dtype));
+  const int32_t odt = out_code(out_dtype);
+  const hipStream_t stream = c10::hip::getCurrentHIPStream(x2.device().index()).stream();
+  const int64_t esz = y.element_size();
+  for (int64_t r0 = 0; r0 < M; r0 += kPromptRows) {
+    const int64_t rows = std::min(kPromptRows, M - r0);
+    const void* xr = static_cast<const uint16_t*>(x2.data_ptr()) + r0 * K;
+    void* yr = static_cast<char*>(y.data_ptr()) + r0 * n * esz;
+    const int64_t ws = pp ? mtl_w4_gemm_prefill_gather_workspace_bytes(rows, K, n)
+                          : mtl_w4_gemm_prefill_workspace_bytes(rows, K, n);
+    at::Tensor wsb = at::empty({ws}, x2.options().dtype(at::kByte));
+    void* wp = ws > 0 ? wsb.data_ptr() : nullptr;
+    if (pp) {
+      check_status(mtl_w4_gemm_prefill_gather(xr, rows, K, K, pp, w.data_ptr<int32_t>(),
+                                              sc.data_ptr(), z.data_ptr<int32_t>(), n,
+                                              (int32_t)group_size, (int32_t)zero_offset, odt, yr, n,
+                                              wp, ws, stream),
+                   "mtl_w4_gemm_prefill_gather");
+    } else {
+      check_status(mtl_w4_gemm_prefill(xr, rows, K, K, w.data_ptr<int32_t>(), sc.data_ptr(),
+                                       z.data_ptr<int32_t>(), n, (int32_t)group_size,
+                                       (int32_t)zero_offset, MTL_EPI_NONE, odt, yr, n,
+                                       static_cast<float*>(wp), ws, stream),
+                   "mtl_w4_gemm_prefill");
+    }
+  }
+  return y.view(out_shape(x, n));
+}
+
 at::Tensor strip_gemv_meta(const at::Tensor& x, const at::Tensor& strip_weight,
                            const at::Tensor& strip_scales, const at::Tensor& strip_zeros,
                            int64_t n, int64_t group_size, int64_t zero_offset,
@@ -293,6 +357,9 @@ TORCH_LIBRARY(mtl, m) {
   m.def("strip_gemv(Tensor x, Tensor strip_weight, Tensor strip_scales, Tensor strip_zeros, "
         "int n, int group_size, int zero_offset=0, Tensor? perm=None, "
         "ScalarType out_dtype=bfloat16) -> Tensor");
+  m.def("prompt_gemm(Tensor x, Tensor strip_weight, Tensor strip_scales, Tensor strip_zeros, "
+        "int n, int group_size, int zero_offset=0, Tensor? perm=None, "
+        "ScalarType out_dtype=bfloat16) -> Tensor");
 }
 
 TORCH_LIBRARY_IMPL(mtl, CUDA, m) {
@@ -301,6 +368,7 @@ TORCH_LIBRARY_IMPL(mtl, CUDA, m) {
   m.impl("gptq_gemm", &gptq_gemm);
   m.impl("strip_rows_gemm", &strip_rows_gemm);
   m.impl("strip_gemv", &strip_gemv);
+  m.impl("prompt_gemm", &prompt_gemm);
 }
 
 TORCH_LIBRARY_IMPL(mtl, Meta, m) {
@@ -309,4 +377,5 @@ TORCH_LIBRARY_IMPL(mtl, Meta, m) {
   m.impl("gptq_gemm", &gptq_gemm_meta);
   m.impl("strip_rows_gemm", &strip_rows_gemm_meta);
   m.impl("strip_gemv", &strip_gemv_meta);
+  m.impl("prompt_gemm", &strip_gemv_meta);
 }

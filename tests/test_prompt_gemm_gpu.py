@@ -162,3 +162,43 @@ def test_embed_rows_unaligned_table(dev):
             v = t[i] if 0 <= i < 30 else torch.zeros_like(t[0])
             h = v if h is None else h + v
         assert torch.equal(out[r], h)
+
+
+@pytest.mark.parametrize("m,k,n,g,act", [
+    (17, 512, 128, 32, True), (40, 768, 256, 256, True), (65, 4096, 384, 64, True),
+    (200, 1024, 1024, 128, True), (33, 12288, 128, 128, True), (100, 1024, 256, 128, False),
+])
+def test_gptq_module_prompt_rows(dev, m, k, n, g, act):
+    # more than 16 rows run on the prompt-length GEMM: against float64, equal to the C entry on
+    # the gathered x, for a strided batch, and inside a graph captured before the first call
+    from moss_tts_lite_amd.gptq import GPTQLinear
+    from oracle import synth
+    from tests.test_gemm_gpu import TOL_F32, rel_l2, t_bf16, t_f16, t_i32
+
+    case = synth.gptq_case(k=k, n=n, m=m, group=g, act_order=act, seed=m + k + n)
+
+    def linear():
+        return GPTQLinear.from_buffers(t_i32(case["qweight"], dev), t_i32(case["qzeros"], dev),
+                                       t_f16(case["scales"], dev),
+                                       t_i32(case["g_idx"], dev) if act else None, g).post_init()
+
+    lin, x = linear(), t_bf16(case["x_bits"], dev)
+    y = lin(x, out_dtype=torch.float32)
+    assert rel_l2(y.cpu().numpy(), case["y_ref"]) < TOL_F32
+    xg = x if lin.perm is None else x.index_select(1, lin.perm.long())
+    sc, qz = lin.strip_meta()
+    assert torch.equal(y, ops.prefill_gemm(xg, lin._strip, sc, qz, n, g, out_dtype=torch.float32))
+    wide = torch.zeros(m, k + 3, dtype=torch.bfloat16, device=dev)
+    wide[:, 1:k + 1] = x
+    assert torch.equal(lin(wide[:, 1:k + 1], out_dtype=torch.float32), y)
+    assert lin(x.reshape(1, m, k)).shape == (1, m, n)
+    fresh = linear()                              # captured before any eager call
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = fresh(x, out_dtype=torch.float32)
+    assert fresh._strip is None
+    for _ in range(2):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(out.cpu().numpy(), case["y_ref"]) < TOL_F32
+        assert torch.equal(fresh(x, out_dtype=torch.float32), y)
