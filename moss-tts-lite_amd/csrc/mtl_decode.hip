@@ -404,7 +404,6 @@ struct AttnArgs {
   int H, Hkv;
   int64_t max_seq;
   float scale, eps;
-  int fixed_chunks;           // chunks are the fixed blocks [64c, 64c + 64)
 };
 
 
@@ -485,214 +484,25 @@ __device__ __forceinline__ void attn_merge(const AttnArgs& a, int kvh, int nch, 
   }
 }
 
-template <bool FROM_PART>
-__global__ void __launch_bounds__(256) attn_decode_kernel(AttnArgs a) {
-  constexpr int D = 128;
-  __shared__ u32x4 q_lds[kAttnMaxRep][16];
-  __shared__ u32x4 kpos[16], vpos[16];
-  __shared__ float e_lds[4][kAttnBlock];
-  __shared__ __attribute__((aligned(16))) float w_lds[4][kAttnMaxChunks];
-  __shared__ int last_flag;
-  const int kvh = blockIdx.x, c = blockIdx.y;
-  const int wave = wave_id(), lane = threadIdx.x & 63;
-  const int n_rep = a.H / a.Hkv;
-  // 0. The q|k|v partials of this wave's first q head (and, on waves 0/1, of this kv
-  //    head's k or v) do not depend on the position: in flight before it is read.
-  const int ncols = (a.H + 2 * a.Hkv) * D;
-  HeadPart hq, hkv;
-  if (FROM_PART && wave < n_rep)
-    head_issue(a.qkv_part, a.splits, ncols, kvh * n_rep + wave, lane, hq);
-  const uint16_t* kbase = a.kc + (size_t)kvh * a.max_seq * D;
-  const uint16_t* vbase = a.vc + (size_t)kvh * a.max_seq * D;
-  const int dg = lane & 15, ps = lane >> 4;           // value pass: dims 8dg.., positions ps+4i
-  u32x4 kr[16], vr[16];
-  // K rows and V slices of positions [base, base + 64) of this kv head, clamped to `last`
-  // (a position in the cache)
-  auto load_k = [&](int base, int last) {
-    const int pk = base + lane < last ? base + lane : last;
-    const u32x4* krow = reinterpret_cast<const u32x4*>(kbase + (size_t)pk * D);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) kr[i] = krow[i];
-  };
-  auto load_v = [&](int base, int last) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int pv = base + ps + 4 * i < last ? base + ps + 4 * i : last;
-      vr[i] = *reinterpret_cast<const u32x4*>(vbase + (size_t)pv * D + 8 * dg);
-    }
-  };
-  // With max_seq <= 64 * 64 every chunk is the fixed block [64c, 64c + 64), so its K rows
-  // load before the position is known (rows at or past the length are masked); V, needed
-  // only after the scores, waits for the position (chunks past the length load nothing
-  // more).
-  const bool fixed = a.fixed_chunks;
-  if (fixed) load_k(c * kAttnBlock, (int)a.max_seq - 1);
-  const int64_t pos = *a.pos;
-  int64_t L64 = pos + 1;
-  if (L64 < 0) L64 = 0;
-  if (L64 > a.max_seq) L64 = a.max_seq;
-  const int L = (int)L64;
-  int nch = (L + kAttnBlock - 1) / kAttnBlock;
-  if (nch > kAttnMaxChunks) nch = kAttnMaxChunks;
-  if (c >= nch) return;                               // uniform over the workgroup
-  const int clen = fixed ? kAttnBlock : (L + nch - 1) / nch;
-  const int p0 = c * clen;
-  const int p1 = p0 + clen < L ? p0 + clen : L;       // p0 < p1 unless the chunk is empty
-  const bool has_pos = pos >= p0 && pos < p1;
-
-  // 1. The first block's V slices (and, unless fixed, K rows), before the q prologue.
-  auto load_block = [&](int base) {
-    load_k(base, p1 - 1 > 0 ? p1 - 1 : 0);
-    load_v(base, p1 - 1 > 0 ? p1 - 1 : 0);
-  };
-  if (fixed) load_v(p0, p1 - 1 > 0 ? p1 - 1 : 0);
-  else if (p0 < p1) load_block(p0);
-  if (FROM_PART && has_pos && wave < 2)   // k (wave 0) or v (wave 1) of position pos
-    head_issue(a.qkv_part, a.splits, ncols, (wave == 0 ? a.H : a.H + a.Hkv) + kvh, lane, hkv);
-
-  // 2. Prologue: q heads into LDS; k/v of position pos (cache + LDS) where it is scored.
-  const size_t prow = (size_t)(pos >= 0 && pos < a.max_seq ? pos : 0) * D;
-  if (FROM_PART) {
-    const uint16_t* cr = a.cos_tab + prow;
-    const uint16_t* sr = a.sin_tab + prow;
-    if (has_pos && wave < 2) {
-      float x0, x1;
-      head_sum(a.qkv_part, a.splits, ncols, (wave == 0 ? a.H : a.H + a.Hkv) + kvh, lane, hkv,
-               x0, x1);
-      if (wave == 0) norm_rope_pair(x0, x1, a.kn, cr, sr, lane, a.eps, x0, x1);
-      const uint32_t b0 = f32_to_bf16(x0), b1 = f32_to_bf16(x1);
-      uint16_t* dst = (wave == 0 ? a.kc : a.vc) + ((size_t)kvh * a.max_seq + pos) * D;
-      dst[lane] = (uint16_t)b0;
-      dst[lane + 64] = (uint16_t)b1;
-      uint16_t* l16 = reinterpret_cast<uint16_t*>(wave == 0 ? kpos : vpos);
-      l16[lane] = (uint16_t)b0;
-      l16[lane + 64] = (uint16_t)b1;
-    }
-    for (int hr = wave; hr < n_rep; hr += 4) {
-      float x0, x1;
-      if (hr != wave) head_issue(a.qkv_part, a.splits, ncols, kvh * n_rep + hr, lane, hq);
-      head_sum(a.qkv_part, a.splits, ncols, kvh * n_rep + hr, lane, hq, x0, x1);
-      norm_rope_pair(x0, x1, a.qn, cr, sr, lane, a.eps, x0, x1);
-      uint16_t* l16 = reinterpret_cast<uint16_t*>(q_lds[hr]);
-      l16[lane] = (uint16_t)f32_to_bf16(x0);
-      l16[lane + 64] = (uint16_t)f32_to_bf16(x1);
-    }
-  } else {
-    for (int hr = wave; hr < n_rep; hr += 4)
-      if (lane < 16)
-        q_lds[hr][lane] =
-            reinterpret_cast<const u32x4*>(a.q + (size_t)(kvh * n_rep + hr) * D)[lane];
-    if (has_pos && wave < 2 && lane < 16)   // the cache already holds k/v of pos
-      (wave == 0 ? kpos : vpos)[lane] =
-          reinterpret_cast<const u32x4*>((wave == 0 ? kbase : vbase) + (size_t)pos * D)[lane];
-  }
-  __syncthreads();
-
-  // 3. Scores, softmax and the value sum, one 64-position block at a time.
-  for (int hr = wave; hr < n_rep; hr += 4) {
-    const int h = kvh * n_rep + hr;
-    float m = -INFINITY, l = 0.f;
-    float o[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = 0.f;
-    for (int base = p0; base < p1; base += kAttnBlock) {
-      if (base != p0 || hr != wave) load_block(base);
-      const int p = base + lane;
-      float acc = 0.f;
-      if (p == pos) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) kr[i] = kpos[i];
-      }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const u32x4 qq = q_lds[hr][i];
-        acc = dot2_bf16(kr[i].x, qq.x, acc);
-        acc = dot2_bf16(kr[i].y, qq.y, acc);
-        acc = dot2_bf16(kr[i].z, qq.z, acc);
-        acc = dot2_bf16(kr[i].w, qq.w, acc);
-      }
-      const float s = p < p1 ? acc * a.scale : -INFINITY;
-      const float mn = fmaxf(m, wave_max(s));
-      const float e = p < p1 ? expf(s - mn) : 0.f;
-      const float corr = expf(m - mn);
-      l = fmaf(l, corr, wave_sum(e));
-#pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] *= corr;
-      m = mn;
-      // the value sum takes e rounded to bf16, the sum l the unrounded e: the form of
-      // torch's fused SDPA on bf16 tensors (moss_tts_lite/model.py:183-189)
-      e_lds[wave][(lane & 3) * 16 + (lane >> 2)] = round_bf16(e);   // position ps+4i at ps*16+i
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float ei = e_lds[wave][ps * 16 + i];
-        const int pv = base + ps + 4 * i;
-        const u32x4 v = pv == pos ? vpos[dg] : pv < p1 ? vr[i] : u32x4{0u, 0u, 0u, 0u};
-        const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          o[2 * j] = fmaf(ei, lo_bf(w4[j]), o[2 * j]);
-          o[2 * j + 1] = fmaf(ei, hi_bf(w4[j]), o[2 * j + 1]);
-        }
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      o[j] += __shfl_xor(o[j], 16);
-      o[j] += __shfl_xor(o[j], 32);
-    }
-    // publish (m, l, o) with agent-scope stores: visible to the merging workgroup on
-    // any XCD without a whole-L2 writeback
-    float* ph = a.part + ((size_t)h * kAttnMaxChunks + c) * kAttnPart;
-    if (lane == 0) {
-      __hip_atomic_store(ph, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(ph + 1, l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (lane < 16) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        __hip_atomic_store(ph + 4 + 8 * dg + j, o[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
-
-  // 4. The last workgroup of this kv head merges its q heads' chunks in chunk order.
-  // The count is a release (every partial store of the workgroup happens before it, through
-  // the barrier) and the workgroup that makes it complete takes an acquire fence before any
-  // thread reads the partials: the hand-off is ordered by the memory model, not only by the
-  // store acknowledgements.
-  __builtin_amdgcn_s_waitcnt(0);      // every partial store acknowledged before the count
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    last_flag = __hip_atomic_fetch_add(&a.counters[kvh], 1u, __ATOMIC_RELEASE,
-                                       __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(nch - 1);
-    if (last_flag) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  }
-  __syncthreads();
-  if (!last_flag) return;
-  if (threadIdx.x == 0)
-    __hip_atomic_store(&a.counters[kvh], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  attn_merge<false>(a, kvh, nch, n_rep, wave, lane, w_lds);
-}
-
 // ----------------------------------------------------------------------------------
-// Tile form of the decode attention, for max_seq <= 64 * 64: chunk c is the fixed block
-// [64c, 64c + 64) of positions.  The workgroup loads the chunk's K and V rows once, before
-// the position is read, and stages them in LDS.  Wave w scores positions 16w .. 16w+15
+// Decode attention: chunk c is the fixed block [64c, 64c + 64) of positions, and with a cache
+// of more than 64 * 64 positions (LONG) the blocks 64 (c + 64 i) too, one after the other with
+// a running maximum: which rows a chunk reads never depends on the length, so the workgroup
+// loads its first block's K and V rows before the position is read, and the next block's
+// while one is worked on.  Each block is staged in LDS.  Wave w scores positions 16w .. 16w+15
 // against every q head of the kv head with four v_mfma_f32_16x16x32_bf16 (A = K rows,
 // B = the q heads as columns).  The chunk softmax max and sum meet across the 4 waves
 // in LDS, and O^T = V^T E^T runs on MFMA with the V^T operand read from the V rows by
 // ds_read_b64_tr_b16 (a wave per 32 dims, every q head at once).  Every cross-lane step of
 // this kernel (q/k RMSNorm, softmax, the merge) runs on the VALU (permlane swaps and DPP,
 // mtl_common.h) instead of ds_bpermute: the same bits, about 0.5 us less per launch in the
-// decode step.  The published (m, l, o[128]) per q head and the merge are those of
-// attn_decode_kernel.
+// decode step.
+//
+// LONG: bound by the two memory latencies of a chunk and the merge; 6000 positions x 8 kv heads
+// (24.6 MB) 15.8 us, where a lane per position (K rows read 256 bytes apart, each q head of a
+// kv head loading the block again) took 31 us.
 // ----------------------------------------------------------------------------------
-template <bool FROM_PART, bool LOCAL>
+template <bool FROM_PART, bool LOCAL, bool LONG>
 __global__ void __launch_bounds__(256) attn_tile_kernel(AttnArgs a) {
   constexpr int D = 128, P = kAttnBlock;
   typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -705,6 +515,7 @@ __global__ void __launch_bounds__(256) attn_tile_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) float e_lds[kAttnMaxRep][P];   // exp(s - m), bf16 values
   __shared__ float red_m[4][16], red_l[4][16];  // per-wave max / sum per q head
   __shared__ __attribute__((aligned(16))) float w_lds[4][kAttnMaxChunks];
+  __shared__ u32x4 kpos[LONG ? 16 : 1], vpos[LONG ? 16 : 1];   // k and v of position pos
   __shared__ int last_flag;
   const int kvh = blockIdx.x, c = blockIdx.y;
   const int t = threadIdx.x, wave = wave_id(), lane = t & 63;
@@ -724,24 +535,30 @@ __global__ void __launch_bounds__(256) attn_tile_kernel(AttnArgs a) {
   const uint16_t* vbase = a.vc + (size_t)kvh * a.max_seq * D;
   const int last_row = (int)a.max_seq - 1;
   u32x4 kv[4], vv[4];
+  auto load_rows = [&](int base) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int item = t + 256 * j;
-    int p = c * P + (item >> 4);
-    p = p < last_row ? p : last_row;
-    kv[j] = *reinterpret_cast<const u32x4*>(kbase + (size_t)p * D + 8 * (item & 15));
-    vv[j] = *reinterpret_cast<const u32x4*>(vbase + (size_t)p * D + 8 * (item & 15));
-  }
+    for (int j = 0; j < 4; ++j) {
+      const int item = t + 256 * j;
+      int p = base + (item >> 4);
+      p = p < last_row ? p : last_row;
+      kv[j] = *reinterpret_cast<const u32x4*>(kbase + (size_t)p * D + 8 * (item & 15));
+      vv[j] = *reinterpret_cast<const u32x4*>(vbase + (size_t)p * D + 8 * (item & 15));
+    }
+  };
+  load_rows(c * P);
   const int64_t pos = *a.pos;
   int64_t L64 = pos + 1;
   if (L64 < 0) L64 = 0;
   if (L64 > a.max_seq) L64 = a.max_seq;
   const int L = (int)L64;
-  const int nch = (L + P - 1) / P;
+  int nch = (L + P - 1) / P;
+  if (LONG && nch > kAttnMaxChunks) nch = kAttnMaxChunks;
   if (c >= nch) return;                               // uniform over the workgroup
-  const int p0 = c * P;
-  const int p1 = p0 + P < L ? p0 + P : L;
-  const bool has_pos = pos >= p0 && pos < p1;
+  constexpr int kStride = P * kAttnMaxChunks;         // LONG: positions to the chunk's next block
+  int p0 = c * P;
+  int p1 = p0 + P < L ? p0 + P : L;
+  const bool has_pos = LONG ? pos >= 0 && pos < L && (pos / P) % kAttnMaxChunks == c
+                            : pos >= p0 && pos < p1;
 
   // 1. Prologue: q heads into LDS; k/v of position pos into the cache and the LDS tile.
   const size_t prow = (size_t)(pos >= 0 && pos < a.max_seq ? pos : 0) * D;
@@ -760,7 +577,8 @@ __global__ void __launch_bounds__(256) attn_tile_kernel(AttnArgs a) {
       uint16_t* dst = (wave == 0 ? a.kc : a.vc) + ((size_t)kvh * a.max_seq + pos) * D;
       dst[lane] = (uint16_t)b0;
       dst[lane + 64] = (uint16_t)b1;
-      uint16_t* l16 = reinterpret_cast<uint16_t*>((wave == 0 ? k_lds : v_lds)[pos - p0]);
+      uint16_t* l16 = reinterpret_cast<uint16_t*>(
+          LONG ? (wave == 0 ? kpos : vpos) : (wave == 0 ? k_lds : v_lds)[LONG ? 0 : pos - p0]);
       l16[lane] = (uint16_t)b0;
       l16[lane + 64] = (uint16_t)b1;
     }
@@ -782,138 +600,172 @@ __global__ void __launch_bounds__(256) attn_tile_kernel(AttnArgs a) {
             reinterpret_cast<const u32x4*>(a.q + (size_t)(kvh * n_rep + hr) * D)[lane];
   }
   for (int i = n_rep * 16 + t; i < 16 * 16; i += 256) q_lds[i >> 4][i & 15] = u32x4{0u, 0u, 0u, 0u};
-  // the chunk's rows; rows at or past the length are zero, and the row of pos comes from
-  // the prologue when it computed k/v there
+  float m_run = -INFINITY, l_run = 0.f;         // LONG: of q head lane % 16 over the blocks so far
+  f4 o_run[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  if (LONG) __syncthreads();                    // kpos, vpos
+  while (true) {
+    // the chunk's rows; rows at or past the length are zero, and the row of pos comes from
+    // the prologue when it computed k/v there
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int item = t + 256 * j;
-    const int row = item >> 4, p = p0 + row;
-    if (FROM_PART && p == pos) continue;
-    const u32x4 z{0u, 0u, 0u, 0u};
-    k_lds[row][item & 15] = p < p1 ? kv[j] : z;
-    v_lds[row][item & 15] = p < p1 ? vv[j] : z;
-  }
-  __syncthreads();
-
-  // 2. Scores s[p][h] = K[p] . q[h] on MFMA; lane l holds positions 16w + 4(l/16) + r of
-  //    q head l%16.  Chunk softmax: max and sum per head across the 4 waves.
-  f4 S = {0.f, 0.f, 0.f, 0.f};
-  u32x4 ka[4], qb[4];                           // all 8 operand reads in flight at once
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    ka[k] = k_lds[16 * wave + (lane & 15)][4 * k + (lane >> 4)];
-    qb[k] = q_lds[lane & 15][4 * k + (lane >> 4)];
-  }
-  __builtin_amdgcn_sched_barrier(0);            // keep the scheduler from re-pairing them
-#pragma unroll
-  for (int k = 0; k < 4; ++k)
-    S = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ka[k]),
-                                                __builtin_bit_cast(bf16x8, qb[k]), S, 0, 0, 0);
-  const int hd = lane & 15, g = lane >> 4;
-  float sv[4], mloc = -INFINITY;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int p = p0 + 16 * wave + 4 * g + r;
-    sv[r] = p < p1 ? S[r] * a.scale : -INFINITY;
-    mloc = fmaxf(mloc, sv[r]);
-  }
-  mloc = xor16_max(mloc);                       // cross-lane steps on the VALU
-  mloc = xor32_max(mloc);
-  if (g == 0) red_m[wave][hd] = mloc;
-  __syncthreads();
-  const float M = fmaxf(fmaxf(red_m[0][hd], red_m[1][hd]), fmaxf(red_m[2][hd], red_m[3][hd]));
-  float lsum = 0.f;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float e = expf(sv[r] - M);                  // 0 for masked positions
-    // value sum over bf16(e), sum over e: torch's fused SDPA form (model.py:183-189)
-    if (hd < n_rep) e_lds[hd][16 * wave + 4 * g + r] = round_bf16(e);
-    lsum += e;
-  }
-  lsum = xor16_add(lsum);
-  lsum = xor32_add(lsum);
-  if (g == 0) red_l[wave][hd] = lsum;
-  __syncthreads();
-
-  // 3. O^T (dims x q heads) = V^T (dims x positions) E^T (positions x heads) on MFMA:
-  //    wave w takes dims 32w .. 32w+31 (two 16-dim blocks) for every q head at once.  The
-  //    A operand V^T comes straight from the V rows in LDS through ds_read_b64_tr_b16: in
-  //    each 16-lane group, lane j reads 4 dims (4(j%4) ..) of position row j/4, and the
-  //    transpose hands lane i dim i of those 4 rows; two reads give a lane its 8
-  //    positions.  B = E^T: lane (g, hd) packs the bf16 probabilities (rounded above) of
-  //    head hd at its 8 positions.  Then publish (m, l, o).
-  {
-    typedef short s4 __attribute__((ext_vector_type(4)));
-    const int hd2 = lane & 15, g2 = lane >> 4;
-    bf16x8 eb[2];                                  // B operands of the two 32-position steps
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const float* er = &e_lds[hd2 < n_rep ? hd2 : 0][32 * ks + 8 * g2];
-      const float4 e0 = reinterpret_cast<const float4*>(er)[0];
-      const float4 e1 = reinterpret_cast<const float4*>(er)[1];
-      const float ev[8] = {e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w};
-      u32x4 w;
-      uint32_t* wp = reinterpret_cast<uint32_t*>(&w);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        wp[i] = hd2 < n_rep ? (__float_as_uint(ev[2 * i]) >> 16) |
-                                  (__float_as_uint(ev[2 * i + 1]) & 0xffff0000u)
-                            : 0u;
-      eb[ks] = __builtin_bit_cast(bf16x8, w);
-    }
-    // this lane's transpose-read addresses: row j/4 of its 8-row step, dims 4(j%4) ..
-    const int jr = (lane & 15) >> 2, jc = 4 * (lane & 3);
-    f4 acc[2];
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb) {
-      const int d0 = 32 * wave + 16 * mb + jc;     // first of this lane's 4 dims
-      s4 rv[2][2];
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-        for (int hf = 0; hf < 2; ++hf) {
-          const int row = 32 * ks + 8 * g2 + 4 * hf + jr;
-          const uint16_t* src = reinterpret_cast<const uint16_t*>(v_lds[row]) + d0;
-          rv[ks][hf] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (s4 __attribute__((address_space(3)))*)(src));
+    for (int j = 0; j < 4; ++j) {
+      const int item = t + 256 * j;
+      const int row = item >> 4, p = p0 + row;
+      const u32x4 z{0u, 0u, 0u, 0u};
+      if (FROM_PART && p == pos) {
+        if (LONG) {
+          k_lds[row][item & 15] = kpos[LONG ? item & 15 : 0];
+          v_lds[row][item & 15] = vpos[LONG ? item & 15 : 0];
         }
-      acc[mb] = f4{0.f, 0.f, 0.f, 0.f};
+        continue;
+      }
+      k_lds[row][item & 15] = p < p1 ? kv[j] : z;
+      v_lds[row][item & 15] = p < p1 ? vv[j] : z;
+    }
+    const bool more = LONG && p0 + kStride < L;   // uniform over the workgroup
+    if (more) load_rows(p0 + kStride);
+    __syncthreads();
+
+    // 2. Scores s[p][h] = K[p] . q[h] on MFMA; lane l holds positions 16w + 4(l/16) + r of
+    //    q head l%16.  Chunk softmax: max and sum per head across the 4 waves.
+    f4 S = {0.f, 0.f, 0.f, 0.f};
+    u32x4 ka[4], qb[4];                           // all 8 operand reads in flight at once
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      ka[k] = k_lds[16 * wave + (lane & 15)][4 * k + (lane >> 4)];
+      qb[k] = q_lds[lane & 15][4 * k + (lane >> 4)];
+    }
+    __builtin_amdgcn_sched_barrier(0);            // keep the scheduler from re-pairing them
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      S = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ka[k]),
+                                                  __builtin_bit_cast(bf16x8, qb[k]), S, 0, 0, 0);
+    const int hd = lane & 15, g = lane >> 4;
+    float sv[4], mloc = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int p = p0 + 16 * wave + 4 * g + r;
+      sv[r] = p < p1 ? S[r] * a.scale : -INFINITY;
+      mloc = fmaxf(mloc, sv[r]);
+    }
+    mloc = xor16_max(mloc);                       // cross-lane steps on the VALU
+    mloc = xor32_max(mloc);
+    if (g == 0) red_m[wave][hd] = mloc;
+    __syncthreads();
+    float M = fmaxf(fmaxf(red_m[0][hd], red_m[1][hd]), fmaxf(red_m[2][hd], red_m[3][hd]));
+    float corr = 1.f;
+    if (LONG) {
+      M = fmaxf(M, m_run);
+      corr = expf(m_run - M);                     // 0 at the first block
+      m_run = M;
+    }
+    float lsum = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float e = expf(sv[r] - M);                  // 0 for masked positions
+      // value sum over bf16(e), sum over e: torch's fused SDPA form (model.py:183-189)
+      if (hd < n_rep) e_lds[hd][16 * wave + 4 * g + r] = round_bf16(e);
+      lsum += e;
+    }
+    lsum = xor16_add(lsum);
+    lsum = xor32_add(lsum);
+    if (g == 0) red_l[wave][hd] = lsum;
+    __syncthreads();
+
+    // 3. O^T (dims x q heads) = V^T (dims x positions) E^T (positions x heads) on MFMA:
+    //    wave w takes dims 32w .. 32w+31 (two 16-dim blocks) for every q head at once.  The
+    //    A operand V^T comes straight from the V rows in LDS through ds_read_b64_tr_b16: in
+    //    each 16-lane group, lane j reads 4 dims (4(j%4) ..) of position row j/4, and the
+    //    transpose hands lane i dim i of those 4 rows; two reads give a lane its 8
+    //    positions.  B = E^T: lane (g, hd) packs the bf16 probabilities (rounded above) of
+    //    head hd at its 8 positions.  Then publish (m, l, o).
+    {
+      typedef short s4 __attribute__((ext_vector_type(4)));
+      const int hd2 = lane & 15, g2 = lane >> 4;
+      bf16x8 eb[2];                                  // B operands of the two 32-position steps
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        const s4 lo = rv[ks][0], hi = rv[ks][1];
-        const bf16x8 A = __builtin_bit_cast(
-            bf16x8, (short __attribute__((ext_vector_type(8)))){lo[0], lo[1], lo[2], lo[3],
-                                                                 hi[0], hi[1], hi[2], hi[3]});
-        acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, eb[ks], acc[mb], 0, 0, 0);
+        const float* er = &e_lds[hd2 < n_rep ? hd2 : 0][32 * ks + 8 * g2];
+        const float4 e0 = reinterpret_cast<const float4*>(er)[0];
+        const float4 e1 = reinterpret_cast<const float4*>(er)[1];
+        const float ev[8] = {e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w};
+        u32x4 w;
+        uint32_t* wp = reinterpret_cast<uint32_t*>(&w);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          wp[i] = hd2 < n_rep ? (__float_as_uint(ev[2 * i]) >> 16) |
+                                    (__float_as_uint(ev[2 * i + 1]) & 0xffff0000u)
+                              : 0u;
+        eb[ks] = __builtin_bit_cast(bf16x8, w);
       }
-    }
-    // acc[mb][r]: dim 32w + 16mb + 4g2 + r of q head hd2
-    if (hd2 < n_rep) {
-      float* ph = a.part + ((size_t)(kvh * n_rep + hd2) * kAttnMaxChunks + c) * kAttnPart;
-      if (wave == 0 && g2 == 0) {
-        const float mh = fmaxf(fmaxf(red_m[0][hd2], red_m[1][hd2]), fmaxf(red_m[2][hd2], red_m[3][hd2]));
-        const float lh = (red_l[0][hd2] + red_l[1][hd2]) + (red_l[2][hd2] + red_l[3][hd2]);
-        if (LOCAL) {
-          *reinterpret_cast<float2*>(ph) = make_float2(mh, lh);
-        } else {
-          __hip_atomic_store(ph, mh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          __hip_atomic_store(ph + 1, lh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
+      // this lane's transpose-read addresses: row j/4 of its 8-row step, dims 4(j%4) ..
+      const int jr = (lane & 15) >> 2, jc = 4 * (lane & 3);
+      f4 acc[2];
 #pragma unroll
       for (int mb = 0; mb < 2; ++mb) {
-        float* po = ph + 4 + 32 * wave + 16 * mb + 4 * g2;
-        if (LOCAL) {
-          // plain stores: they end in this XCD's L2, where the merging workgroup reads them
-          *reinterpret_cast<float4*>(po) =
-              make_float4(acc[mb][0], acc[mb][1], acc[mb][2], acc[mb][3]);
-        } else {
+        const int d0 = 32 * wave + 16 * mb + jc;     // first of this lane's 4 dims
+        s4 rv[2][2];
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            __hip_atomic_store(po + r, acc[mb][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+          for (int hf = 0; hf < 2; ++hf) {
+            const int row = 32 * ks + 8 * g2 + 4 * hf + jr;
+            const uint16_t* src = reinterpret_cast<const uint16_t*>(v_lds[row]) + d0;
+            rv[ks][hf] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (s4 __attribute__((address_space(3)))*)(src));
+          }
+        acc[mb] = f4{0.f, 0.f, 0.f, 0.f};
+        if (LONG) acc[mb] = o_run[mb] * corr;     // head lane % 16, as m_run
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          const s4 lo = rv[ks][0], hi = rv[ks][1];
+          const bf16x8 A = __builtin_bit_cast(
+              bf16x8, (short __attribute__((ext_vector_type(8)))){lo[0], lo[1], lo[2], lo[3],
+                                                                   hi[0], hi[1], hi[2], hi[3]});
+          acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, eb[ks], acc[mb], 0, 0, 0);
+        }
+      }
+      if (LONG) {
+        l_run = fmaf(l_run, corr, (red_l[0][hd2] + red_l[1][hd2]) + (red_l[2][hd2] + red_l[3][hd2]));
+        o_run[0] = acc[0];
+        o_run[1] = acc[1];
+        if (more) {
+          p0 += kStride;
+          p1 = p0 + P < L ? p0 + P : L;
+          __syncthreads();                        // every wave is done with this block's LDS
+          continue;
+        }
+      }
+      // acc[mb][r]: dim 32w + 16mb + 4g2 + r of q head hd2
+      if (hd2 < n_rep) {
+        float* ph = a.part + ((size_t)(kvh * n_rep + hd2) * kAttnMaxChunks + c) * kAttnPart;
+        if (wave == 0 && g2 == 0) {
+          const float mh = LONG ? m_run : fmaxf(fmaxf(red_m[0][hd2], red_m[1][hd2]),
+                                                fmaxf(red_m[2][hd2], red_m[3][hd2]));
+          const float lh = LONG ? l_run : (red_l[0][hd2] + red_l[1][hd2]) + (red_l[2][hd2] + red_l[3][hd2]);
+          if (LOCAL) {
+            *reinterpret_cast<float2*>(ph) = make_float2(mh, lh);
+          } else {
+            __hip_atomic_store(ph, mh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(ph + 1, lh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+        }
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb) {
+          float* po = ph + 4 + 32 * wave + 16 * mb + 4 * g2;
+          if (LOCAL) {
+            // plain stores: they end in this XCD's L2, where the merging workgroup reads them
+            *reinterpret_cast<float4*>(po) =
+                make_float4(acc[mb][0], acc[mb][1], acc[mb][2], acc[mb][3]);
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              __hip_atomic_store(po + r, acc[mb][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
         }
       }
     }
+
+    break;
   }
 
   // 4. The last workgroup of this kv head merges its q heads' chunks in chunk order.
@@ -954,8 +806,10 @@ __global__ void __launch_bounds__(256) attn_tile_kernel(AttnArgs a) {
     attn_merge<true, true>(a, kvh, nch, n_rep, wave, lane, w_lds);
     return;
   }
-  // Agent-scope hand-off (release count, acquire fence of the completing workgroup, as in
-  // attn_decode_kernel).
+  // Agent-scope hand-off.  The count is a release (every partial store of the workgroup happens
+  // before it, through the barrier) and the workgroup that makes it complete takes an acquire
+  // fence before any thread reads the partials: the hand-off is ordered by the memory model,
+  // not only by the store acknowledgements.
   if (t == 0) {
     last_flag = __hip_atomic_fetch_add(&a.counters[kvh], 1u, __ATOMIC_RELEASE,
                                        __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(nch - 1);
@@ -1310,25 +1164,20 @@ int mtl_decode_attention_set_handoff(int32_t local) {
 static void attn_launch(AttnArgs& a, void* workspace, bool from_part, hipStream_t s) {
   a.counters = static_cast<uint32_t*>(workspace);
   a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + kAttnCounterBytes);
-  a.fixed_chunks = a.max_seq <= kAttnBlock * kAttnMaxChunks;   // the tile kernel where it fits
   int64_t ch = (a.max_seq + kAttnBlock - 1) / kAttnBlock;
   if (ch > kAttnMaxChunks) ch = kAttnMaxChunks;
   const dim3 grid(a.Hkv, (unsigned)ch);
   // the XCD-local hand-off needs every chunk of a kv head on one XCD: kv heads a multiple
   // of 8, so linear ids kvh + Hkv * c agree modulo 8
   const bool local = g_attn_local_handoff && a.Hkv % 8 == 0 && a.Hkv <= kAttnMaxKvLocal;
-  if (a.fixed_chunks) {
-    if (from_part) {
-      if (local) hipLaunchKernelGGL((attn_tile_kernel<true, true>), grid, dim3(256), 0, s, a);
-      else hipLaunchKernelGGL((attn_tile_kernel<true, false>), grid, dim3(256), 0, s, a);
-    } else {
-      if (local) hipLaunchKernelGGL((attn_tile_kernel<false, true>), grid, dim3(256), 0, s, a);
-      else hipLaunchKernelGGL((attn_tile_kernel<false, false>), grid, dim3(256), 0, s, a);
-    }
-  } else if (from_part) {
-    hipLaunchKernelGGL(attn_decode_kernel<true>, grid, dim3(256), 0, s, a);
+  const bool lng = a.max_seq > kAttnBlock * kAttnMaxChunks;
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, a); };
+  if (from_part) {
+    if (lng) local ? go(attn_tile_kernel<true, true, true>) : go(attn_tile_kernel<true, false, true>);
+    else local ? go(attn_tile_kernel<true, true, false>) : go(attn_tile_kernel<true, false, false>);
   } else {
-    hipLaunchKernelGGL(attn_decode_kernel<false>, grid, dim3(256), 0, s, a);
+    if (lng) local ? go(attn_tile_kernel<false, true, true>) : go(attn_tile_kernel<false, false, true>);
+    else local ? go(attn_tile_kernel<false, true, false>) : go(attn_tile_kernel<false, false, false>);
   }
 }
 

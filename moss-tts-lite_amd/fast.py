@@ -687,10 +687,15 @@ class FastDecoder:
     def _wide_bytes(self, rows: int, lin) -> int:
         """Workspace bytes of the dequantised-operand GEMM where ``lin`` runs ``rows`` prompt
         rows on it (mtl_w4_gemm_prompt_qsz: plain x in, no split partials), else 0."""
-        if lin.stream_weight(True)[1] != N.LAYOUT_STRIP_QSZ:
+        if not isinstance(lin, QszLinear):
             return 0
-        return int(N.load().mtl_w4_gemm_prompt_qsz_workspace_bytes(
-            rows, lin.in_features, lin.out_features, lin.group_size))
+        memo = self._pf.setdefault("wide_bytes", {})
+        key = (rows, lin.in_features, lin.out_features, lin.group_size)
+        if key not in memo:
+            if len(memo) > 256:      # many prompt lengths
+                memo.clear()
+            memo[key] = int(N.load().mtl_w4_gemm_prompt_qsz_workspace_bytes(*key))
+        return memo[key]
 
     def _prefill_wide(self, x, rows: int, lin, epilogue: int, y, ldy: int, stream) -> None:
         """One prompt-length GEMM of the reference's records on plain x
