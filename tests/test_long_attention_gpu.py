@@ -66,3 +66,41 @@ def test_long_cache_attention(dev, H, Hkv, max_seq, positions, local):
             assert not ws[:1024].any()           # counters back at zero, placement held
     finally:
         lib.mtl_decode_attention_set_handoff(1)
+
+
+# row blocks past one and two turns of the deal (32 blocks of 16 rows), a ragged last block, both
+# group counts (4 and 8 q heads per kv head), fewer tiles than wave groups
+@pytest.mark.parametrize("H,Hkv,L,pos0", [(8, 2, 530, 0), (4, 1, 1100, 3), (16, 2, 545, 0),
+                                          (8, 2, 19, 61), (4, 4, 65, 0)])
+def test_prefill_attention_rows(dev, H, Hkv, L, pos0):
+    gen = torch.Generator(device=dev).manual_seed(L)
+    S = pos0 + L + 5
+    kc, vc = (torch.randn(Hkv, S, 128, device=dev, generator=gen).bfloat16() for _ in range(2))
+    kc[:, S - 5:] = float("nan")                 # rows past the prompt are not read into a result
+    vc[:, S - 5:] = float("nan")
+    q = torch.randn(L, H * 128, device=dev, generator=gen).bfloat16()
+    out = torch.zeros(L, H * 128, dtype=torch.bfloat16, device=dev)
+    N.check(N.load().mtl_prefill_attention(
+        q.data_ptr(), kc.data_ptr(), vc.data_ptr(), L, pos0, out.data_ptr(), H * 128, None, H, Hkv,
+        128, S, ctypes.c_float(128 ** -0.5), torch.cuda.current_stream().cuda_stream), "attention")
+    torch.cuda.synchronize()
+    n = pos0 + L
+    k, v = (c[:, :n].double().repeat_interleave(H // Hkv, 0) for c in (kc, vc))
+    s = q.double().reshape(L, H, 128).transpose(0, 1) @ k.transpose(1, 2) * 128 ** -0.5
+    keep = torch.arange(n, device=dev)[None] <= pos0 + torch.arange(L, device=dev)[:, None]
+    ref = (torch.softmax(s.masked_fill(~keep, float("-inf")), -1) @ v).transpose(0, 1).reshape(L, -1)
+    err = (out.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    assert float(err.max()) < 1e-2               # bf16 probabilities and output
+    # through an output index, 16-byte aligned and not, and with rows 2 bytes off: the same values
+    perm = torch.randperm(H * 128, device=dev, generator=gen).int()
+    for ix, ld, off in ((perm, None, 0), (None, H * 128 + 1, 1),
+                        (torch.cat([perm[:1], perm])[1:], None, 0)):
+        ld = ld or H * 128
+        buf = torch.zeros(L * ld + off, dtype=torch.bfloat16, device=dev)
+        N.check(N.load().mtl_prefill_attention(
+            q.data_ptr(), kc.data_ptr(), vc.data_ptr(), L, pos0, buf[off:].data_ptr(), ld,
+            None if ix is None else ix.data_ptr(), H, Hkv, 128, S, ctypes.c_float(128 ** -0.5),
+            torch.cuda.current_stream().cuda_stream), "attention")
+        torch.cuda.synchronize()
+        got = buf[off:].reshape(L, ld)[:, :H * 128]
+        assert torch.equal(got if ix is None else got[:, ix.long()], out)
