@@ -31,7 +31,6 @@ typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 
 constexpr int kWdStrips = 4;                     // 16-column strips per wave
-constexpr int kWdKW = 2;                         // K halves (wave groups) of a workgroup
 constexpr int kWdCols = 4 * kWdStrips * 16;      // 256 columns per workgroup
 constexpr int kWdMaxRT = 6;                      // 16-row tiles per workgroup: 144 KB of LDS
 constexpr int kXTop = 6, kWTop = 13;             // binades of the row and column maxima
@@ -228,9 +227,12 @@ __device__ __forceinline__ void dequant_step(uint32_t w, u32x4& t, uint32_t lo, 
   asm volatile("" : "+v"(t.x), "+v"(t.y), "+v"(t.z), "+v"(t.w));   // keeps the step here
 }
 
-// A workgroup (8 waves, one per CU and two per SIMD) owns RT row tiles x 256 columns; wave
-// (kg, wn) multiplies all RT tiles by 64 columns (4 strips) over half kg of the K blocks, and
-// the two halves meet in LDS at the end.  RT = 6 is what three x buffers leave of the LDS: a
+// A workgroup owns RT row tiles x 256 columns; wave (kg, wn) multiplies all RT tiles by 64
+// columns (4 strips) over part kg of the K blocks.  Either way two waves share a SIMD: KW = 2 is
+// a workgroup of 8 waves per CU whose two halves of K meet in LDS at the end, for grids that
+// would not give every CU two workgroups; KW = 1 two independent workgroups of 4 waves, whose
+// barriers do not hold each other up (1100 x 4096 x 24576: 308 -> 289 us at g = 32, 265 -> 235
+// at g = 128; 389 rows 129 -> 119; but 1100 x 12288 x 4096, 224 workgroups: 159 -> 200).  RT = 6 is what three x buffers leave of the LDS: a
 // dequantised operand (12 VALU instructions per 8 codes) feeds 6 MFMAs and an x operand 4.
 // The x tiles come by direct loads into LDS two turns ahead (the staged order is the operand
 // order, so there is no conversion and no bank conflict), weights and scales into registers
@@ -264,13 +266,13 @@ __device__ __forceinline__ void wait_and_barrier() {
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-template <int RT, int MB>
-__global__ void __launch_bounds__(256 * kWdKW) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <int RT, int MB, int KW>
+__global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 w4_wide_kernel(WideArgs a) {
   // x tiles of three turns, [tile][chunk of the block][lane] (one tile more at an odd RT, for
   // the halves' exchange at the end)
   constexpr int kBuf = (RT + 1) / 2 * 512;
-  __shared__ u32x4 xa[3][kWdKW][kBuf];
+  __shared__ u32x4 xa[3][KW][kBuf];
   const int lane = threadIdx.x & 63, wave = wave_id();
   const int kg = wave >> 2, wn = wave & 3;
   const int lg = lane >> 4, lj = lane & 15;
@@ -300,7 +302,7 @@ w4_wide_kernel(WideArgs a) {
       const_cast<u32x4*>(a.zf), (short)0, (int)((int64_t)(N / 16) * a.zchunks * 1024), 0x00020000);
 
   // strips past N read zeros (outside the buffers) and are not stored
-  const int b0 = kg * (kb >> 1), nblk = kb >> 1; // this wave group's blocks (kb is even)
+  const int nblk = kb / KW, b0 = kg * nblk;      // this wave group's blocks (kb is even)
   u32x4 wq[3][kWdStrips];
   u32x2 mq[3][kWdStrips];                        // its scales, packed f16 (MB = 4: both words)
   auto issue_w = [&](int r, int i) {             // block i of the group's (clamped)
@@ -330,7 +332,7 @@ w4_wide_kernel(WideArgs a) {
     int off = (4 * b + wn) * 1024;
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
-      lds_load16(xres, lds0 + (uint32_t)((r * kWdKW * kBuf + 256 * t) * 16), lane * 16, off);
+      lds_load16(xres, lds0 + (uint32_t)((r * KW * kBuf + 256 * t) * 16), lane * 16, off);
       if (t + 1 < nrt) off += tstep;
     }
   };
@@ -348,7 +350,7 @@ w4_wide_kernel(WideArgs a) {
     for (int s = 0; s < kWdStrips; ++s) acc[tt][s] = zero4;
 
   // zeros: sum over the groups of z * X, 32 groups per MFMA, X in three parts
-  for (int c = kg; c < a.zchunks; c += kWdKW) {
+  for (int c = kg; c < a.zchunks; c += KW) {
     f16x8_t Z[kWdStrips];
 #pragma unroll
     for (int s = 0; s < kWdStrips; ++s)
@@ -448,23 +450,25 @@ w4_wide_kernel(WideArgs a) {
   }
   wait_and_barrier<0>();                         // no load into LDS is left
 
-  // The halves meet: wave group kg keeps tiles of its parity and hands over the others.
+  // KW = 2: the halves meet, wave group kg keeping tiles of its half and handing over the others.
   // acc[tt][s][i] is column 16 (strip0 + s) + 4 lg + i of row 16 (mt0 + tt) + lj.
   constexpr int H0 = (RT + 1) / 2;               // group 0 keeps tiles 0 .. H0 - 1
-  floatx4* mine = reinterpret_cast<floatx4*>(&xa[kg][0][0]);
-  floatx4* theirs = reinterpret_cast<floatx4*>(&xa[1 - kg][0][0]);
+  const floatx4* theirs = reinterpret_cast<const floatx4*>(&xa[KW == 2 ? 1 - kg : 0][0][0]);
+  if constexpr (KW == 2) {
+    floatx4* mine = reinterpret_cast<floatx4*>(&xa[kg][0][0]);
 #pragma unroll
-  for (int tt = 0; tt < RT; ++tt)
-    if ((tt >= H0) == (kg == 0)) {
-      const int slot = tt >= H0 ? tt - H0 : tt;
+    for (int tt = 0; tt < RT; ++tt)
+      if ((tt >= H0) == (kg == 0)) {
+        const int slot = tt >= H0 ? tt - H0 : tt;
 #pragma unroll
-      for (int s = 0; s < kWdStrips; ++s)
-        mine[((wn * H0 + slot) * kWdStrips + s) * 64 + lane] = acc[tt][s];
-    }
-  __syncthreads();
+        for (int s = 0; s < kWdStrips; ++s)
+          mine[((wn * H0 + slot) * kWdStrips + s) * 64 + lane] = acc[tt][s];
+      }
+    __syncthreads();
+  }
 #pragma unroll
   for (int tt = 0; tt < RT; ++tt) {
-    if ((tt >= H0) != (kg == 1)) continue;
+    if (KW == 2 && (tt >= H0) != (kg == 1)) continue;
     if (tt >= nrt) continue;
     const int slot = tt >= H0 ? tt - H0 : tt;
     const int row = 16 * (mt0 + tt) + lj;
@@ -472,7 +476,8 @@ w4_wide_kernel(WideArgs a) {
     float v[kWdStrips][4];
 #pragma unroll
     for (int s = 0; s < kWdStrips; ++s) {
-      const floatx4 o = theirs[((wn * H0 + slot) * kWdStrips + s) * 64 + lane];
+      const floatx4 o =
+          KW == 2 ? theirs[((wn * H0 + slot) * kWdStrips + s) * 64 + lane] : zero4;
       const int col = 16 * (strip0 + s) + 4 * lg;
       const int4 ce = *reinterpret_cast<const int4*>(a.cexp + (col < N ? col : 0));
       const int c4[4] = {ce.x, ce.y, ce.z, ce.w};
@@ -608,13 +613,13 @@ bool wide_pays(int64_t M, int64_t K, int64_t N, int32_t group) {
   return false;
 }
 
-template <int MB>
+template <int MB, int KW>
 static void wide_launch(const WideArgs& a, dim3 grid, int rt, hipStream_t st) {
-  const dim3 block(256 * kWdKW);
+  const dim3 block(256 * KW);
   switch (rt) {
-    case 6: hipLaunchKernelGGL((w4_wide_kernel<6, MB>), grid, block, 0, st, a); break;
-    case 5: hipLaunchKernelGGL((w4_wide_kernel<5, MB>), grid, block, 0, st, a); break;
-    default: hipLaunchKernelGGL((w4_wide_kernel<4, MB>), grid, block, 0, st, a); break;
+    case 6: hipLaunchKernelGGL((w4_wide_kernel<6, MB, KW>), grid, block, 0, st, a); break;
+    case 5: hipLaunchKernelGGL((w4_wide_kernel<5, MB, KW>), grid, block, 0, st, a); break;
+    default: hipLaunchKernelGGL((w4_wide_kernel<4, MB, KW>), grid, block, 0, st, a); break;
   }
 }
 
@@ -663,9 +668,10 @@ int wide_gemm(const void* x, int64_t M, int64_t ldx, int64_t K, const int32_t* s
   a.nb = wide_row_blocks(rtiles, ctiles, pf_device_cus());
   const int rt = (int)((rtiles + a.nb - 1) / a.nb);
   const dim3 grid((unsigned)(a.nb * ctiles));
-  if (s.mb == 1) wide_launch<1>(a, grid, rt, st);
-  else if (s.mb == 2) wide_launch<2>(a, grid, rt, st);
-  else wide_launch<4>(a, grid, rt, st);
+  const bool two = 2 * (int64_t)grid.x < 3 * pf_device_cus();   // one workgroup for most CUs
+  if (s.mb == 1) two ? wide_launch<1, 2>(a, grid, rt, st) : wide_launch<1, 1>(a, grid, rt, st);
+  else if (s.mb == 2) two ? wide_launch<2, 2>(a, grid, rt, st) : wide_launch<2, 1>(a, grid, rt, st);
+  else two ? wide_launch<4, 2>(a, grid, rt, st) : wide_launch<4, 1>(a, grid, rt, st);
   return launch_status();
 }
 
