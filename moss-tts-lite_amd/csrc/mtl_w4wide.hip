@@ -12,8 +12,8 @@
 // MFMA contraction over 3 K / g (9 % of the main one at g = 32, 2 % at 128).
 //
 // Measured, both launches, against mtl_w4prefill.hip on one chip: 389 x 4096 x 24576 at g = 32
-// 171 -> 104 us (755 TFLOP/s), 1100 x 4096 x 24576 at g = 32 401 -> 280 us, 1536 x 12288 x 4096
-// at g = 128 193 -> 159 us (975 TFLOP/s; a large bf16 matrix product of the library reaches
+// 171 -> 96 us (815 TFLOP/s), 1100 x 4096 x 24576 at g = 32 440 -> 265 us, 1536 x 12288 x 4096
+// at g = 128 193 -> 155 us (995 TFLOP/s; a large bf16 matrix product of the library reaches
 // 1450 here).
 //
 // Range.  A launch before the GEMM (wide_stage_kernel) finds a power of two per row of x and
@@ -73,11 +73,12 @@ __device__ __forceinline__ uint32_t pk_f16(float a, float b) {
 }
 
 // One launch per GEMM: the first rowblocks workgroups stage x, 256 threads per row; the others
-// reduce and stage the columns' metadata, 64 columns each.  Bound by memory latency: 9.5 us at
-// 389 x 4096 and 24576 columns at g = 32 (6.4 MB of x, 25 MB of metadata), 28 us at
-// 1536 x 12288 (75 MB).  With a wave per row and 2-byte metadata stores the first took 16.8 us.
+// reduce and stage the columns' metadata, 64 columns each.  Bound by memory latency: 8.6 us at
+// 389 x 4096 and 24576 columns at g = 32 (6.4 MB of x, 25 MB of metadata), 24 us at
+// 1536 x 12288 (75 MB); with the row read again for its second use 9.5 and 28, and with a wave
+// per row and 2-byte metadata stores the first took 16.8.
 //
-// A row is read twice (the second time from L2): its largest magnitude, then its f16 values
+// A row is used twice: for its largest magnitude, then for its f16 values
 // in the order of the MFMA operand: chunk c of 32 channels of row tile t is 1 KB, lane l
 // holding row l % 16, channels 32 c + 8 (l / 16) .. + 7 in the pair order of the codes.  The
 // four rows of a workgroup are neighbours, so their 16-byte pieces fill 64-byte segments.
@@ -154,14 +155,21 @@ __global__ void __launch_bounds__(1024) wide_stage_kernel(StageArgs a) {
   const int items = K >> 3;                      // 8-channel items; a multiple of 32
   const bool live = row < a.M;                   // rows of the last tile past M stage zeros
   const u32x4* xr = reinterpret_cast<const u32x4*>(a.x + (size_t)(live ? row : a.M - 1) * a.ldx);
+  // The row's first 8 x 256 items stay in registers (K <= 16384: all), the rest is read again.
+  u32x4 xv[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+    if (256 * c < items) xv[c] = xr[t4 + 256 * c < items ? t4 + 256 * c : 0];
   uint32_t mx = 0;
-#pragma unroll 4
-  for (int i = t4; i < items; i += 256) {
-    const u32x4 v = xr[i];
+  auto take = [&](const u32x4& v) {
     const uint32_t e[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int j = 0; j < 4; ++j) mx = max(mx, max(e[j] & 0x7fffu, (e[j] >> 16) & 0x7fffu));
-  }
+  };
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+    if (256 * c < items) take(xv[c]);            // item 0 again where there is none
+  for (int i = 2048 + t4; i < items; i += 256) take(xr[i]);
   red[wave][lane] = mx;
   __syncthreads();
 #pragma unroll
@@ -182,11 +190,8 @@ __global__ void __launch_bounds__(1024) wide_stage_kernel(StageArgs a) {
       X -= f16_to_f32(h);
     }
   };
-#pragma unroll 4
-  for (int i0 = 0; i0 < items; i0 += 256) {
-    const int i = i0 + t4;
+  auto put = [&](u32x4 v, int i) {
     const bool in = i < items;                   // whole groups are in or out
-    u32x4 v = xr[in ? i : 0];
     if (!live) v = u32x4{0, 0, 0, 0};
     float sum;
     const u32x4 pv = pair_order_dot(v, sum);
@@ -202,7 +207,11 @@ __global__ void __launch_bounds__(1024) wide_stage_kernel(StageArgs a) {
     if (per > 8) sum += dpp_f32<kDppMirror>(sum);
     if (per > 16) sum = xor16_add(sum);
     if (in && (i & (per - 1)) == 0) zput(i / per, ldexpf(sum, ex));
-  }
+  };
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+    if (256 * c < items) put(xv[c], t4 + 256 * c);
+  for (int i0 = 2048; i0 < items; i0 += 256) put(xr[i0 + t4 < items ? i0 + t4 : 0], i0 + t4);
   for (int g = a.ngroups + t4; g < 32 * a.zchunks; g += 256) zput(g, 0.f);
 }
 

@@ -54,7 +54,7 @@ def rel(a, b):
 @pytest.mark.parametrize("m,k,n,g", [
     (1, 256, 16, 32), (16, 512, 256, 256), (17, 768, 272, 128), (33, 1792, 336, 64),
     (65, 1024, 1040, 32), (97, 4608, 256, 256), (389, 1024, 4096, 32), (600, 512, 5120, 128),
-    (1100, 768, 4096, 64), (1536, 512, 4096, 128),
+    (1100, 768, 4096, 64), (1536, 512, 4096, 128), (21, 16640, 64, 128),
     # grids of workgroups that take all of K (1.5 workgroups per CU and more): 2 and 6 blocks,
     # a ragged last column tile, 4, 5 and 6 row tiles
     (420, 256, 24592, 128), (200, 768, 24576, 64), (389, 512, 24576, 32), (576, 256, 18432, 256),
