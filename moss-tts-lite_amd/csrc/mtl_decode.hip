@@ -320,14 +320,10 @@ __global__ void __launch_bounds__(64) qk_norm_rope_kv_kernel(
 
 // ----------------------------------------------------------------------------------
 // GQA decode attention over positions [0, pos] (fast.py:149-162), split over the
-// sequence.  Grid (kv head, chunk): nch = min(ceil(L / 64), 64) chunks of at most
-// ceil(L / nch) positions, so for L <= 4096 a workgroup scores at most 64 positions in
-// one pass with every K and V load in flight at once.  Wave w of a workgroup serves q
-// head kvh * n_rep + w (+4, ...).  Scores are lane-per-position dot products against the
-// wave-uniform q; the value sum gives each lane 8 dims of 16 positions (u32x4 loads),
-// reduced across the 4 position groups at the end.  Each chunk publishes
-// (max, sum, o[128]); the last workgroup of a kv head to finish (agent-scope counter)
-// merges that head group's chunks in chunk order, so there is no second launch.
+// sequence.  Grid (kv head, chunk): nch = min(ceil(L / 64), 64) chunks of 64-position blocks
+// (attn_tile_kernel).  Each chunk publishes (max, sum, o[128]); the last workgroup of a kv
+// head to finish merges that head group's chunks in chunk order, so there is no second
+// launch.
 // With FROM_PART, q/k RMSNorm, RoPE and the KV write of position pos run in the
 // prologue from the q|k|v split-K partials (fast.py:134-147); the workgroup holding pos
 // uses its LDS copy of k/v for that position.

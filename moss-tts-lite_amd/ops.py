@@ -160,7 +160,8 @@ def weight_int4pack_mm(x: torch.Tensor, packed: torch.Tensor, q_group_size: int,
     ``qScaleAndZeros`` bf16 ``[K/g, N, 2]`` = (scale, zero) with
     ``w = (q - 8) * scale + zero`` (moss_tts_lite/gptq.py:87-97).  Returns bf16 ``[M, N]``.
     M = 1 runs the full-K strip GEMV, 2 to 16 rows the skinny strip GEMM, more
-    rows the prompt-length GEMM.  ``RuntimeError`` for a wrong shape, dtype or group size,
+    rows the prompt-length GEMM or, from 64 rows where it is faster, the GEMM with
+    dequantised operands.  ``RuntimeError`` for a wrong shape, dtype or group size,
     as torch's operator raises.
     """
     return torch_ops().weight_int4pack_mm(x, packed, q_group_size, q_scale_and_zeros)
