@@ -12,7 +12,7 @@
 // MFMA contraction over 3 K / g (9 % of the main one at g = 32, 2 % at 128).
 //
 // Measured, both launches, against mtl_w4prefill.hip on one chip: 389 x 4096 x 24576 at g = 32
-// 171 -> 96 us (815 TFLOP/s), 1100 x 4096 x 24576 at g = 32 440 -> 265 us, 1536 x 12288 x 4096
+// 171 -> 96 us (815 TFLOP/s), 1100 x 4096 x 24576 at g = 32 401 -> 249 us, 1536 x 12288 x 4096
 // at g = 128 193 -> 155 us (995 TFLOP/s; a large bf16 matrix product of the library reaches
 // 1450 here).
 //
@@ -602,11 +602,11 @@ static double other_us(int64_t M, int64_t K, int64_t N, int32_t group, int cus) 
 
 // Measured (us, this GEMM against the other, both launches of each; 256 CUs):
 //   K x N, g          M = 96        192          389           600            1100
-//   4096 x 24576, 32  49 / 55     62 / 89     106 / 172     157 / 230      280 / 401
-//   4096 x 24576, 128 40 / 41     52 / 66      92 / 123     139 / 165      246 / 284
-//   12288 x 4096, 32 105 / 33    108 / 44     114 / 97      117 / 128      156 / 221
-//   4096 x 4096, 128  38 / 18     40 / 23      44 / 34       45 / 40        56 / 64
-//   1024 x 2000, 32   19 / 29     21 / 58      21 / 121      22 / 185       25 / 337
+//   4096 x 24576, 32  49 / 55     60 / 89      99 / 172     143 / 230      249 / 401
+//   4096 x 24576, 128 40 / 41     51 / 66      85 / 123     126 / 165      221 / 284
+//   12288 x 4096, 32 105 / 33    108 / 44     114 / 97      117 / 128      140 / 221
+//   4096 x 4096, 128  38 / 18     40 / 23      44 / 34       45 / 40        52 / 64
+//   1024 x 2000, 32   19 / 29     20 / 58      21 / 121      22 / 185       24 / 337
 // so the line lies where the estimates cross, with a tenth in hand, from 64 rows on.
 bool wide_pays(int64_t M, int64_t K, int64_t N, int32_t group) {
   if (M < 64 || M > (1 << 20) || K < 256 || K % 256 != 0 || K > 65536 || N < 16 || N % 16 != 0)
