@@ -24,6 +24,7 @@
 // under the rounding of the fp32 sums.  X, the fp32 sum of a group's x, enters as three f16
 // parts.
 #include "mtl_w4core.h"
+#include "mtl_w4wide_reads.h"
 
 namespace mtl {
 
@@ -310,7 +311,10 @@ w4_wide_kernel(WideArgs a) {
   const __amdgpu_buffer_rsrc_t zrsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<u32x4*>(a.zf), (short)0, (int)((int64_t)(N / 16) * a.zchunks * 1024), 0x00020000);
 
-  // strips past N read zeros (outside the buffers) and are not stored
+  // strips past N repeat the last one and are not stored
+  int strip[kWdStrips];
+#pragma unroll
+  for (int s = 0; s < kWdStrips; ++s) strip[s] = wide_strip(strip0 + s, N / 16);
   const int nblk = kb / KW, b0 = kg * nblk;      // this wave group's blocks (kb is even)
   u32x4 wq[3][kWdStrips];
   u32x2 mq[3][kWdStrips];                        // its scales, packed f16 (MB = 4: both words)
@@ -318,17 +322,17 @@ w4_wide_kernel(WideArgs a) {
     const int b = b0 + (i < nblk ? i : nblk - 1);
 #pragma unroll
     for (int s = 0; s < kWdStrips; ++s) {
-      const int rec = (strip0 + s) * a.krec + (a.krec == kb ? b : b >> 1);   // g = 256: pairs
+      const int at = wide_scale_at(strip[s], a.krec, kb, b, MB);
       if (MB == 4) {
         mq[r][s] = __builtin_bit_cast(
-            u32x2, __builtin_amdgcn_raw_buffer_load_b64(srsrc, lj * 8, rec * 128, 0));
+            u32x2, __builtin_amdgcn_raw_buffer_load_b64(srsrc, lj * 8, at, 0));
       } else if (MB == 2) {
-        mq[r][s].x = __builtin_amdgcn_raw_buffer_load_b32(srsrc, lj * 4, rec * 64, 0);
+        mq[r][s].x = __builtin_amdgcn_raw_buffer_load_b32(srsrc, lj * 4, at, 0);
       } else {
-        mq[r][s].x = __builtin_amdgcn_raw_buffer_load_b16(srsrc, lj * 2, rec * 32, 0);
+        mq[r][s].x = __builtin_amdgcn_raw_buffer_load_b16(srsrc, lj * 2, at, 0);
       }
       wq[r][s] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                               wrsrc, lane * 16, ((strip0 + s) * kb + b) * 1024, 0));
+                                               wrsrc, lane * 16, wide_weight_at(strip[s], kb, b), 0));
     }
   };
   constexpr int kLoadsW = 2 * kWdStrips;         // loads of one issue_w (in order, as issued)
@@ -364,7 +368,7 @@ w4_wide_kernel(WideArgs a) {
 #pragma unroll
     for (int s = 0; s < kWdStrips; ++s)
       Z[s] = __builtin_bit_cast(f16x8_t, __builtin_amdgcn_raw_buffer_load_b128(
-          zrsrc, lane * 16, ((strip0 + s) * a.zchunks + c) * 1024, 0));
+          zrsrc, lane * 16, wide_zero_at(strip[s], a.zchunks, c), 0));
     const int k0 = (a.K >> 5) + 3 * c;
 #pragma unroll
     for (int tt = 0; tt < RT; ++tt) {
@@ -611,7 +615,7 @@ static double other_us(int64_t M, int64_t K, int64_t N, int32_t group, int cus) 
 bool wide_pays(int64_t M, int64_t K, int64_t N, int32_t group) {
   if (M < 64 || M > (1 << 20) || K < 256 || K % 256 != 0 || K > 65536 || N < 16 || N % 16 != 0)
     return false;
-  const int64_t cols = (N + kWdCols - 1) / kWdCols * kWdCols;   // offsets past N stay in 31 bits
+  const int64_t cols = (N + kWdCols - 1) / kWdCols * kWdCols;   // offsets stay in 31 bits
   if (cols / 16 * (K / 128) * 1024 >= ((int64_t)1 << 31) || cols * (K / 32) * 4 >= ((int64_t)1 << 31))
     return false;
   const int cus = pf_device_cus();
