@@ -24,6 +24,24 @@ __all__ = ["GPTQLinear", "QszLinear", "fuse_gptq_linears", "fuse_qsz_linears",
 LIN_NAMES = ("q", "k", "v", "o", "gate", "up", "down")
 
 
+def _stamp(buffers: dict) -> tuple:
+    """What the copies made from a linear's buffers are valid for: each tensor with its version,
+    which every in-place operation of torch counts up, and whether one of them keeps none (an
+    inference tensor)."""
+    t = [buffers[n] for n in ("qweight", "g_idx", "scales", "qzeros")]
+    v = [None if x.is_inference() else x._version for x in t]
+    return (t[0], v[0], t[1], v[1], t[2], v[2], t[3], v[3], None in v)
+
+
+def _into(dst: torch.Tensor | None, src: torch.Tensor) -> torch.Tensor:
+    """``src`` written into the copy ``dst`` where that has its shape (whoever holds its
+    address then reads the new values), else ``src`` itself."""
+    if dst is None or dst.shape != src.shape or dst.device != src.device or \
+            (dst.is_inference() and not torch.is_inference_mode_enabled()):
+        return src
+    return dst.copy_(src)
+
+
 class GPTQLinear(torch.nn.Module):
     """4-bit GPTQ linear, ``y = x @ dequant(qweight)`` with AutoGPTQ buffers.
 
@@ -56,6 +74,8 @@ class GPTQLinear(torch.nn.Module):
         self._strip_meta: tuple | None = None
         self._strip_only = False
         self._perm16: torch.Tensor | None = None     # the act-order index as int16 (K <= 12288)
+        self._one_row: tuple | None = None           # what the strip GEMV reads of these
+        self._src: tuple | None = None               # _stamp of the buffers they are copies of
 
     @classmethod
     def from_buffers(cls, qweight, qzeros, scales, g_idx=None, group_size: int = 128,
@@ -70,6 +90,13 @@ class GPTQLinear(torch.nn.Module):
             m.g_idx = g_idx.to(device=qweight.device, dtype=torch.int32).contiguous()
         return m
 
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        if "_src" not in state:                      # pickled without: its copies are current
+            self._one_row = None
+            self._src = None if self._kernel_qweight is None and not self._strip_only else \
+                _stamp(self._buffers)
+
     def is_act_order(self) -> bool:
         trivial = torch.arange(self.in_features, device=self.g_idx.device, dtype=torch.int32) \
             // self.group_size
@@ -78,14 +105,63 @@ class GPTQLinear(torch.nn.Module):
     @torch.no_grad()
     def post_init(self) -> "GPTQLinear":
         """Build the kernel-side weight: for act-order, the group-sorted copy and gather index."""
-        if self._strip_only:
-            return self
-        if self.is_act_order():
-            self._kernel_qweight, self._perm = ops.actorder_prepare(self.qweight, self.g_idx,
-                                                                    self.group_size)
-        else:
-            self._kernel_qweight, self._perm = self.qweight, None
+        if not self._strip_only:
+            self._remake(None)
         return self
+
+    def _update(self) -> bool:
+        """Bring the copies up to date with the buffers: they are made again when a buffer was
+        replaced or changed in place since (``load_state_dict``).  False where they are not and
+        cannot be (:meth:`_remake`).  A compiled call reads them as they were when it was
+        compiled."""
+        s, b = self._src, self._buffers
+        if s is not None:
+            if torch.compiler.is_compiling():
+                return True
+            qw, gi, sc, qz = b["qweight"], b["g_idx"], b["scales"], b["qzeros"]
+            if s[0] is qw and s[2] is gi and s[4] is sc and s[6] is qz and \
+                    (s[1] is None or s[1] == qw._version) and \
+                    (s[3] is None or s[3] == gi._version) and \
+                    (s[5] is None or s[5] == sc._version) and \
+                    (s[7] is None or s[7] == qz._version):
+                return True
+        return self._remake(s)
+
+    @torch.no_grad()
+    def _remake(self, old: tuple | None) -> bool:
+        """Make the copies again whose buffers are not those of ``old`` (None: all).  False inside
+        a graph capture, where the new ones would only be filled at replay: the old ones stay."""
+        new = _stamp(self._buffers)
+        same = [old is not None and old[i] is new[i] and old[i + 1] == new[i + 1]
+                for i in (0, 2, 4, 6)]
+        # after drop_original or keep_strip_only the copies are all there is of the weight
+        weight = not (same[0] and same[1]) and not self._strip_only and \
+            (old is None or new[0].numel() > 0)
+        if old is not None and new[4].is_cuda and torch.cuda.is_current_stream_capturing():
+            if weight and self._perm is not None:
+                raise RuntimeError("the weight changed since its kernel copies were made: call "
+                                   "post_init (or run the linear once) before capturing it")
+            return False
+        self._one_row = None
+        if weight:
+            if self.is_act_order():
+                qw, perm = ops.actorder_prepare(self.qweight, self.g_idx, self.group_size)
+                if self._perm is not None:      # else _kernel_qweight is a buffer, not a copy
+                    qw, perm = _into(self._kernel_qweight, qw), _into(self._perm, perm)
+            else:
+                qw, perm = self.qweight, None
+            if self._strip is not None:
+                self._strip = _into(self._strip, ops.strip_weights(qw))
+            if self._tiled is not None:
+                self._tiled = _into(self._tiled, ops.tile_weights(qw))
+            if self._perm16 is not None:
+                self._perm16 = None if perm is None else _into(self._perm16, perm.to(torch.int16))
+            self._kernel_qweight, self._perm = qw, perm
+        if self._strip_meta is not None and not (same[2] and same[3]):
+            sc, qz = ops.strip_meta(self.scales, self.qzeros, self.group_size)
+            self._strip_meta = _into(self._strip_meta[0], sc), _into(self._strip_meta[1], qz)
+        self._src = new
+        return True
 
     def kernel_args(self):
         """``(qweight, qzeros, scales, perm)`` of the AutoGPTQ-layout kernels (the weight
@@ -93,16 +169,16 @@ class GPTQLinear(torch.nn.Module):
         if self._strip_only:
             raise RuntimeError("this linear keeps only its strip copy (keep_strip_only): "
                                "the AutoGPTQ-layout kernels have no weight to read")
-        if self._kernel_qweight is None:
-            self.post_init()
-        return self._kernel_qweight, self.qzeros, self.scales, self._perm
+        self._update()
+        # without act-order the buffer itself: nothing is derived that could be behind it
+        qw = self.qweight if self._perm is None else self._kernel_qweight
+        return qw, self.qzeros, self.scales, self._perm
 
     @property
     def perm(self) -> torch.Tensor | None:
         """The act-order gather index (int32 ``[K]``: sorted row i is input channel
         ``perm[i]``), or None when the groups are contiguous."""
-        if self._kernel_qweight is None and not self._strip_only:
-            self.post_init()
+        self._update()
         return self._perm
 
     @torch.no_grad()
@@ -119,6 +195,7 @@ class GPTQLinear(torch.nn.Module):
         self._kernel_qweight = None
         self._tiled = None
         self.qweight = torch.empty(0, dtype=torch.int32, device=self.scales.device)
+        self._src = _stamp(self._buffers)
         self._strip_only = True
         return self
 
@@ -131,51 +208,65 @@ class GPTQLinear(torch.nn.Module):
 
         ``strip=False``: the wave-contiguous tiled copy of the kernel weight (split-K
         GEMV) when N % 64 == 0, else the kernel weight in row layout.  ``strip=True``:
-        the column-strip copy for the full-K strip GEMV.  Copies are built once."""
-        if strip and self._strip is not None:
+        the column-strip copy for the full-K strip GEMV.  Copies are built once, and again
+        when the buffers change (:meth:`_update`)."""
+        current = self._update()
+        if strip and self._strip is not None and (current or self._strip_only):
             return self._strip, N.LAYOUT_STRIP
         qw = self.kernel_args()[0]
         if strip:
             if not self.supports_strip():
                 raise RuntimeError(f"no strip layout for K={self.in_features}, "
                                    f"N={self.out_features}")
-            self._strip = ops.strip_weights(qw)
-            return self._strip, N.LAYOUT_STRIP
+            copy = ops.strip_weights(qw)
+            if current:
+                self._strip = copy
+            return copy, N.LAYOUT_STRIP
         if self.out_features % 64:
             return qw, N.LAYOUT_ROWS
-        if self._tiled is None:
-            self._tiled = ops.tile_weights(qw)
-        return self._tiled, N.LAYOUT_TILED
+        if self._tiled is not None and current:
+            return self._tiled, N.LAYOUT_TILED
+        copy = ops.tile_weights(qw)
+        if current:
+            self._tiled = copy
+        return copy, N.LAYOUT_TILED
 
     def strip_meta(self):
-        """``(scales, qzeros)`` in the strip order the strip GEMV reads (built once)."""
-        if self._strip_meta is None:
-            self._strip_meta = ops.strip_meta(self.scales, self.qzeros, self.group_size)
-        return self._strip_meta
+        """``(scales, qzeros)`` in the strip order the strip GEMV reads (built once, and again
+        when either buffer changes)."""
+        current = self._update()
+        if self._strip_meta is not None and current:
+            return self._strip_meta
+        meta = ops.strip_meta(self.scales, self.qzeros, self.group_size)
+        if current:
+            self._strip_meta = meta
+        return meta
 
     def _prompt_ready(self, x: torch.Tensor) -> bool:
-        """Whether the prompt-length GEMM can take this linear's rows: the strip layout and
-        whole 128-column tiles, and the strip copy and its metadata there.  They are built at
-        the first such call (not inside a graph capture, where they would only be filled at
-        replay, nor on a tensor that stands for another in a trace) and waited for, so that any
-        stream may read them."""
+        """Whether the prompt-length GEMM takes this linear's rows on the strip copy and its
+        metadata (made at the first such call, and waited for so that any stream may read them).
+        It does not where the AutoGPTQ buffers are read at every call and a copy would not follow
+        them: in a graph capture, a compiled call or on a tensor that stands for another in a
+        trace, and for inference tensors, whose changes leave no mark."""
+        if self.out_features % 128 or not x.is_cuda or torch.compiler.is_compiling() or \
+                type(x) not in (torch.Tensor, torch.nn.Parameter) or self._src[8] or \
+                torch.cuda.is_current_stream_capturing():
+            return False
         if self._strip is None or self._strip_meta is None:
-            if not self.supports_strip() or self.out_features % 128 or \
-                    not self.scales.is_cuda or torch.compiler.is_compiling() or \
-                    type(x) not in (torch.Tensor, torch.nn.Parameter) or \
-                    torch.cuda.is_current_stream_capturing():
+            scales = self._buffers["scales"]
+            if not self.supports_strip() or not scales.is_cuda:
                 return False
-            strip = self._strip if self._strip is not None else \
-                ops.strip_weights(self.kernel_args()[0])
-            meta = self._strip_meta or ops.strip_meta(self.scales, self.qzeros, self.group_size)
-            torch.cuda.current_stream(self.scales.device).synchronize()
-            self._strip, self._strip_meta = strip, meta
-        return self.out_features % 128 == 0
+            self.stream_weight(strip=True)
+            self.strip_meta()
+            torch.cuda.current_stream(scales.device).synchronize()
+        return True
 
     def drop_original(self) -> None:
         """Free the unsorted ``qweight`` once the sorted copy exists (load-time memory)."""
-        if self._perm is not None:
+        if self._perm is not None and not self._strip_only:
+            self._update()
             self.qweight = torch.empty(0, dtype=torch.int32, device=self.qweight.device)
+            self._src = _stamp(self._buffers)
 
     @torch.no_grad()
     def reorder_output_columns(self, cols: torch.Tensor) -> "GPTQLinear":
@@ -190,9 +281,8 @@ class GPTQLinear(torch.nn.Module):
         cols = cols.to(device=self.scales.device, dtype=torch.long)
         if cols.numel() != self.out_features:
             raise ValueError("cols must list every output column once")
-        if self._kernel_qweight is None:
-            self.post_init()
-        self._tiled = self._strip = self._strip_meta = self._perm16 = None
+        self._update()
+        self._tiled = self._strip = self._strip_meta = self._perm16 = self._one_row = None
         sorted_separately = self._kernel_qweight is not self.qweight
         self._kernel_qweight = self._kernel_qweight[:, cols].contiguous()
         if sorted_separately and self.qweight.numel():
@@ -201,6 +291,7 @@ class GPTQLinear(torch.nn.Module):
             self.qweight = self._kernel_qweight
         self.scales = self.scales[:, cols].contiguous()
         self.qzeros = _pack_cols(_unpack_cols(self.qzeros)[:, cols])
+        self._src = _stamp(self._buffers)
         return self
 
     def forward(self, x: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
@@ -208,39 +299,56 @@ class GPTQLinear(torch.nn.Module):
         through the act-order index while staging), few rows on the skinny strip GEMM where
         it pays (:func:`ops.strip_rows_pays`), more than 16 on the prompt-length GEMM (x
         gathered by a launch before it) where N is a multiple of 128; all read the strip copy
-        of the weight, built once and kept.  The others run on the split-K GEMM over the
+        of the weight, built once and kept as long as the buffers stay as they are.  The others run on the split-K GEMM over the
         AutoGPTQ layout, 16 rows at a time (4096 x 24576, g128, act-order: 33 us per 16 rows
         against 30-70 us for 17 to 256 rows on the prompt-length GEMM).  Calls
         go through the ``torch.ops.mtl`` operators (one dispatcher call, torch's stream and
         allocator)."""
         m = x.numel() // self.in_features if self.in_features else 0
-        perm = self.perm
-        if m == 1 and self.supports_strip() and (perm is None or self.in_features <= 12288):
-            strip = self.stream_weight(strip=True)[0]
-            sc, qz = self.strip_meta()
-            if perm is not None and self._perm16 is None:
-                self._perm16 = perm.to(torch.int16)
-            return ops.strip_gemv(x, strip, sc, qz, self.out_features, self.group_size,
-                                  self.zero_offset, self._perm16, out_dtype)
-        if m and self.supports_strip() and (
-                (self._strip_only and m <= 16) or
+        current = self._update()
+        if m == 1:
+            ready = self._one_row if current else None
+            if ready is None:
+                ready = self._one_row_args()
+            if ready is not None:
+                return ops.overload("strip_gemv")(x, ready[0], ready[1], ready[2],
+                                                  self.out_features, self.group_size,
+                                                  self.zero_offset, ready[3], out_dtype)
+        perm = self._perm
+        if 0 < m <= 16 and self.supports_strip() and (
+                self._strip_only or
                 ops.strip_rows_pays(m, self.in_features, self.out_features, perm is not None)):
-            strip = self.stream_weight(strip=True)[0]
-            return ops.torch_ops().strip_rows_gemm(x, strip, self.qzeros, self.scales,
+            strip = self._strip if current else None
+            if strip is None:
+                strip = self.stream_weight(strip=True)[0]
+            b = self._buffers
+            return ops.overload("strip_rows_gemm")(x, strip, b["qzeros"], b["scales"],
                                                    self.out_features, self.group_size,
                                                    self.zero_offset, perm, out_dtype)
-        if self._strip_only:
-            # the prompt-length GEMM is all that is left: it raises where N % 128 != 0
-            sc, qz = self.strip_meta()
-            return ops.torch_ops().prompt_gemm(x, self._strip, sc, qz, self.out_features,
-                                               self.group_size, self.zero_offset, perm, out_dtype)
-        if m > 16 and self._prompt_ready(x):
-            sc, qz = self._strip_meta
-            return ops.torch_ops().prompt_gemm(x, self._strip, sc, qz, self.out_features,
+        # after keep_strip_only the prompt-length GEMM is all that is left: it raises where
+        # N % 128 != 0
+        if self._strip_only or m > 16 and self._prompt_ready(x):
+            sc, qz = self._strip_meta if current else self.strip_meta()
+            return ops.overload("prompt_gemm")(x, self._strip, sc, qz, self.out_features,
                                                self.group_size, self.zero_offset, perm, out_dtype)
         qw, qz, sc, perm = self.kernel_args()
         return ops.gptq_gemm(x, qw, qz, sc, self.group_size, perm=perm,
                              zero_offset=self.zero_offset, out_dtype=out_dtype)
+
+    def _one_row_args(self) -> tuple | None:
+        """``(strip copy, its scales and zeros, int16 gather index)`` of the strip GEMV, kept for
+        the next call; None for a shape that it does not take."""
+        perm = self._perm
+        if not self.supports_strip() or (perm is not None and self.in_features > 12288):
+            return None
+        strip = self.stream_weight(strip=True)[0]
+        sc, qz = self.strip_meta()
+        if perm is not None and self._perm16 is None:
+            self._perm16 = perm.to(torch.int16)
+        ready = strip, sc, qz, self._perm16
+        if strip is self._strip and sc is self._strip_meta[0]:
+            self._one_row = ready
+        return ready
 
     def dequantize(self) -> torch.Tensor:
         """Exact fp32 ``W[K, N]`` in the original input-channel order."""

@@ -1,0 +1,239 @@
+"""When a GPTQ linear's kernel copies are made, kept and made again: the module's own code on the
+CPU, its kernels replaced by plain stand-ins that fill their outputs outside torch's sight, as
+the library does through raw pointers."""
+import ctypes
+import io
+import types
+
+import pytest
+import torch
+
+from moss_tts_lite_amd import gptq, ops
+
+K, N, G = 256, 128, 64
+
+
+def _filled(src):
+    """A copy that only memory knows of: torch sees an empty tensor."""
+    src = src.contiguous()
+    out = torch.empty_like(src)
+    ctypes.memmove(out.data_ptr(), src.data_ptr(), src.numel() * src.element_size())
+    return out
+
+
+def _product(x, qw, qz, sc, g, perm, zo, dt):
+    """x @ dequant(W) of AutoGPTQ-layout tensors, the weight's rows sorted by group."""
+    j = torch.arange(8, dtype=torch.int32) * 4
+    q = ((qw.unsqueeze(1) >> j.view(1, 8, 1)) & 15).reshape(-1, qw.shape[1]).float()
+    z = ((qz.unsqueeze(2) >> j) & 15).reshape(qz.shape[0], -1).float() + zo
+    w = (q - z.repeat_interleave(g, 0)) * sc.float().repeat_interleave(g, 0)
+    xg = x if perm is None else x.index_select(-1, perm.long())
+    return (xg.float() @ w).to(dt)
+
+
+@pytest.fixture
+def kernels(monkeypatch):
+    """The stand-ins and the list of products that ran."""
+    ran = []
+
+    def strip(name):
+        def run(x, w, sc, qz, n, g, zo=0, perm=None, dt=torch.bfloat16):
+            ran.append(name)
+            if name == "rows":
+                sc, qz = qz, sc
+            return _product(x, w, qz, sc, g, perm, zo, dt)
+        return run
+
+    def plain(x, qw, qz, sc, g, perm=None, zo=0, dt=torch.bfloat16):
+        ran.append("gptq")
+        return _product(x, qw, qz, sc, g, perm, zo, dt)
+
+    def actorder(qw, g_idx, g):
+        if g_idx.numel() != qw.shape[0] * 8:
+            raise RuntimeError("g_idx must have K entries")
+        perm = torch.argsort(g_idx, stable=True).int()
+        j = torch.arange(8, dtype=torch.int32) * 4
+        q = ((qw.unsqueeze(1) >> j.view(1, 8, 1)) & 15).reshape(-1, qw.shape[1])[perm.long()]
+        return _filled((q.view(-1, 8, qw.shape[1]) << j.view(1, 8, 1)).sum(1).int()), _filled(perm)
+
+    lib = types.SimpleNamespace(gptq_gemm=plain, strip_gemv=strip("gemv"),
+                                strip_rows_gemm=strip("rows"), prompt_gemm=strip("prompt"))
+    stream = types.SimpleNamespace(synchronize=lambda: None)
+    monkeypatch.setattr(ops, "torch_ops", lambda: lib)
+    monkeypatch.setattr(ops, "overload", lambda name: getattr(lib, name))
+    monkeypatch.setattr(ops, "strip_weights", _filled)
+    monkeypatch.setattr(ops, "strip_meta", lambda sc, qz, g: (_filled(sc), _filled(qz)))
+    monkeypatch.setattr(ops, "actorder_prepare", actorder)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda t: True), raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: stream)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    return ran
+
+
+def _buffers(seed, act):
+    gen = torch.Generator().manual_seed(seed)
+    g_idx = torch.arange(K, dtype=torch.int32) // G
+    return (torch.randint(-2**31, 2**31 - 1, (K // 8, N), dtype=torch.int32, generator=gen),
+            torch.randint(-2**31, 2**31 - 1, (K // G, N // 8), dtype=torch.int32, generator=gen),
+            (torch.rand(K // G, N, generator=gen) * 0.01 + 0.01).half(),
+            g_idx[torch.randperm(K, generator=gen)] if act else None)
+
+
+def _linear(seed, act):
+    return gptq.GPTQLinear.from_buffers(*_buffers(seed, act), G).post_init()
+
+
+def _x(m):
+    return torch.randn(m, K, generator=torch.Generator().manual_seed(m)).bfloat16()
+
+
+ROWS = (1, 4, 40)            # the strip GEMV, the skinny GEMM, the prompt-length GEMM
+
+
+@pytest.mark.parametrize("act", [False, True])
+def test_buffers_changed_after_use(kernels, act):
+    # a linear that has run follows its buffers as a new one does: load_state_dict, an in-place
+    # change of the metadata, replaced tensors
+    for m in ROWS:
+        x = _x(m)
+        lin = _linear(1, act)
+        first = lin(x)
+        lin.load_state_dict(_linear(2, act).state_dict())
+        assert torch.equal(lin(x), _linear(2, act)(x)) and not torch.equal(lin(x), first)
+        lin.scales.mul_(2)
+        assert torch.allclose(lin(x).float(), 2 * _linear(2, act)(x).float(), rtol=1e-2)
+        third = _linear(3, act)
+        lin.qweight, lin.qzeros, lin.scales, lin.g_idx = (t.clone() for t in (
+            third.qweight, third.qzeros, third.scales, third.g_idx))
+        assert torch.equal(lin(x), third(x)), m
+    assert set(kernels) == {"gemv", "rows", "prompt"}
+
+
+def test_copies_are_made_again_in_place(kernels):
+    # a captured graph or a decoder that holds a copy's address reads the new weight through it
+    lin = _linear(1, True)
+    for m in ROWS:
+        lin(_x(m))
+    at = [t.data_ptr() for t in (lin._kernel_qweight, lin._perm, lin._strip, *lin._strip_meta)]
+    lin.load_state_dict(_linear(2, True).state_dict())
+    y = [lin(_x(m)) for m in ROWS]
+    new = [t.data_ptr() for t in (lin._kernel_qweight, lin._perm, lin._strip, *lin._strip_meta)]
+    assert at == new and all(torch.equal(a, _linear(2, True)(_x(m))) for a, m in zip(y, ROWS))
+    made = lin._strip
+    lin(_x(40))
+    assert lin._strip is made
+
+
+def test_dropped_and_reordered_weights_keep_their_copies(kernels):
+    # after drop_original or keep_strip_only the copies are all there is of the weight; the
+    # metadata still follows its buffers
+    x, ref = _x(40), _linear(5, True)(_x(40))
+    lin = _linear(5, True)
+    lin(x)
+    lin.drop_original()
+    assert not lin.qweight.numel() and torch.equal(lin(x), ref)
+    with pytest.raises(RuntimeError):
+        lin.post_init()                              # nothing left to sort, nothing lost
+    assert torch.equal(lin(x), ref)
+    lin.reorder_output_columns(torch.arange(N).flip(0))
+    assert torch.equal(lin(x), ref.flip(-1))
+    lin.keep_strip_only()
+    assert torch.equal(lin(x), ref.flip(-1))
+    lin.scales.mul_(2)
+    assert torch.allclose(lin(x).float(), 2 * ref.flip(-1).float(), rtol=1e-2)
+
+
+def test_a_linear_on_the_host_is_refused():
+    # no stand-ins: the copies' kernels take raw pointers and must not see host memory
+    for act in (False, True):
+        lin = gptq.GPTQLinear.from_buffers(*_buffers(1, act), G)
+        for m in ROWS:
+            with pytest.raises(RuntimeError, match="HIP device|'CPU' backend"):
+                lin(_x(m))
+
+
+def test_changed_inside_a_capture(kernels, monkeypatch):
+    # nothing is kept that only a replay would fill: without act-order the call reads the buffers
+    # or a copy of its own, with it the prepared weight is missing and the call is refused; a
+    # change of the metadata alone needs no weight
+    for act in (False, True):
+        lin = _linear(1, act)
+        for m in ROWS:
+            lin(_x(m))
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+        strip, meta = lin._strip.clone(), lin._strip_meta[0].clone()
+        lin.scales.mul_(2)
+        ref = gptq.GPTQLinear.from_buffers(*_buffers(1, act), G)
+        ref.scales.mul_(2)
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+        want = [ref(_x(m)) for m in ROWS]
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+        assert all(torch.equal(lin(_x(m)), w) for m, w in zip(ROWS, want))
+        lin.load_state_dict(_linear(2, act).state_dict())
+        for m in ROWS:
+            if act:
+                with pytest.raises(RuntimeError, match="before capturing"):
+                    lin(_x(m))
+            else:
+                assert torch.equal(lin(_x(m)), _linear(2, act)(_x(m)))
+        assert torch.equal(lin._strip, strip) and torch.equal(lin._strip_meta[0], meta)
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+        assert all(torch.equal(lin(_x(m)), _linear(2, act)(_x(m))) for m in ROWS)
+
+
+def test_inference_tensors_are_read_at_every_call(kernels):
+    # they keep no version, so a change in place leaves no mark: no copy of them is used for
+    # the rows that were read from the buffers before there was one
+    with torch.inference_mode():
+        lin = _linear(1, False)
+        x = _x(40)
+        first = lin(x)
+        lin.scales.mul_(2)
+        assert torch.allclose(lin(x).float(), 2 * first.float(), rtol=1e-2)
+
+
+def test_saved_modules(kernels):
+    # with the copies and their marks, and as saved before there were marks
+    lin = _linear(1, True)
+    ref = [lin(_x(m)) for m in ROWS]
+    for marked in (True, False):
+        if not marked:
+            del lin._src, lin._one_row
+        buf = io.BytesIO()
+        torch.save(lin, buf)
+        buf.seek(0)
+        back = torch.load(buf, weights_only=False)
+        assert all(torch.equal(back(_x(m)), r) for m, r in zip(ROWS, ref))
+        back.load_state_dict(_linear(2, True).state_dict())
+        assert torch.equal(back(_x(40)), _linear(2, True)(_x(40)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", [False, True])
+def test_buffers_changed_after_use_on_the_device(dev, act):
+    # the kernels themselves, eager and captured: a replay of many rows reads the buffers as
+    # they are, of one row the copy that the eager call brought up to date
+    def linear(seed):
+        return gptq.GPTQLinear.from_buffers(*(None if b is None else b.to(dev)
+                                              for b in _buffers(seed, act)), G).post_init()
+
+    lin, other = linear(1), linear(2)
+    want = {m: other(_x(m).to(dev)) for m in ROWS}
+    graphs = {}
+    for m in ROWS:
+        x = _x(m).to(dev)
+        lin(x)
+        graphs[m] = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graphs[m]):
+            out = lin(x)
+        graphs[m] = graphs[m], out, x
+    lin.load_state_dict(other.state_dict())
+    for m in ROWS:
+        assert torch.equal(lin(_x(m).to(dev)), want[m]), m
+    for _ in range(2):
+        for m, (graph, out, x) in graphs.items():
+            graph.replay()
+            torch.cuda.synchronize()
+            # the captured many-row call runs on the AutoGPTQ layout: other fp32 sums, bf16 out
+            err = (out.float() - want[m].float()).norm() / want[m].float().norm()
+            assert torch.equal(out, want[m]) if m <= 16 else float(err) < 4e-3, (m, float(err))
