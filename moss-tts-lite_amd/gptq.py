@@ -24,6 +24,24 @@ __all__ = ["GPTQLinear", "QszLinear", "fuse_gptq_linears", "fuse_qsz_linears",
 LIN_NAMES = ("q", "k", "v", "o", "gate", "up", "down")
 
 
+# by name: this is asked at every call of a module whose kernels take a few microseconds
+_compiling = torch.compiler.is_compiling
+_jit_tracing = torch._C._is_tracing
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_modes = torch._C._len_torch_function_stack
+_functorch_level = torch._C._functorch.peek_interpreter_stack
+
+
+def _recording() -> bool:
+    """Whether torch's operations are being recorded or transformed (``torch.compile``, export,
+    ``jit.trace``, a dispatch mode as ``make_fx`` or fake tensors enter, ``vmap``).  The kernels
+    that make the copies work on raw pointers, which a recording does not see: it would hold the
+    copy as an uninitialised tensor."""
+    return _compiling() or _jit_tracing() or _dispatch_modes() > 0 or \
+        _functorch_level() is not None or \
+        (_function_modes() > 0 and torch._ops._len_torch_dispatch_stack_pre_dispatch() > 0)
+
+
 def _stamp(buffers: dict) -> tuple:
     """What the copies made from a linear's buffers are valid for: each tensor with its version,
     which every in-place operation of torch counts up, and whether one of them keeps none (an
@@ -130,21 +148,27 @@ class GPTQLinear(torch.nn.Module):
     @torch.no_grad()
     def _remake(self, old: tuple | None) -> bool:
         """Make the copies again whose buffers are not those of ``old`` (None: all).  False inside
-        a graph capture, where the new ones would only be filled at replay: the old ones stay."""
+        a graph capture, where the new ones would only be filled at replay, and where operations
+        are recorded (:func:`_recording`): the old ones stay."""
         new = _stamp(self._buffers)
         same = [old is not None and old[i] is new[i] and old[i + 1] == new[i + 1]
                 for i in (0, 2, 4, 6)]
         # after drop_original or keep_strip_only the copies are all there is of the weight
         weight = not (same[0] and same[1]) and not self._strip_only and \
             (old is None or new[0].numel() > 0)
-        if old is not None and new[4].is_cuda and torch.cuda.is_current_stream_capturing():
+        recording = _recording()
+        if old is not None and (recording or new[4].is_cuda and
+                                torch.cuda.is_current_stream_capturing()):
             if weight and self._perm is not None:
                 raise RuntimeError("the weight changed since its kernel copies were made: call "
-                                   "post_init (or run the linear once) before capturing it")
+                                   "post_init (or run the linear once) before capturing or "
+                                   "tracing it")
             return False
         self._one_row = None
         if weight:
             if self.is_act_order():
+                if recording:
+                    raise RuntimeError("call post_init before tracing an act-order linear")
                 qw, perm = ops.actorder_prepare(self.qweight, self.g_idx, self.group_size)
                 if self._perm is not None:      # else _kernel_qweight is a buffer, not a copy
                     qw, perm = _into(self._kernel_qweight, qw), _into(self._perm, perm)
@@ -246,9 +270,9 @@ class GPTQLinear(torch.nn.Module):
         """Whether the prompt-length GEMM takes this linear's rows on the strip copy and its
         metadata (made at the first such call, and waited for so that any stream may read them).
         It does not where the AutoGPTQ buffers are read at every call and a copy would not follow
-        them: in a graph capture, a compiled call or on a tensor that stands for another in a
-        trace, and for inference tensors, whose changes leave no mark."""
-        if self.out_features % 128 or not x.is_cuda or torch.compiler.is_compiling() or \
+        them: in a graph capture, a trace or compiled call or on a tensor subclass, and for
+        inference tensors, whose changes leave no mark."""
+        if self.out_features % 128 or not x.is_cuda or _recording() or \
                 type(x) not in (torch.Tensor, torch.nn.Parameter) or self._src[8] or \
                 torch.cuda.is_current_stream_capturing():
             return False
@@ -308,17 +332,18 @@ class GPTQLinear(torch.nn.Module):
         current = self._update()
         if m == 1:
             ready = self._one_row if current else None
-            if ready is None:
+            if ready is None and self._strip_allowed():
                 ready = self._one_row_args()
             if ready is not None:
                 return ops.overload("strip_gemv")(x, ready[0], ready[1], ready[2],
                                                   self.out_features, self.group_size,
                                                   self.zero_offset, ready[3], out_dtype)
         perm = self._perm
+        strip = self._strip if current else None
         if 0 < m <= 16 and self.supports_strip() and (
                 self._strip_only or
-                ops.strip_rows_pays(m, self.in_features, self.out_features, perm is not None)):
-            strip = self._strip if current else None
+                ops.strip_rows_pays(m, self.in_features, self.out_features, perm is not None)) \
+                and (strip is not None or self._strip_allowed()):
             if strip is None:
                 strip = self.stream_weight(strip=True)[0]
             b = self._buffers
@@ -334,6 +359,11 @@ class GPTQLinear(torch.nn.Module):
         qw, qz, sc, perm = self.kernel_args()
         return ops.gptq_gemm(x, qw, qz, sc, self.group_size, perm=perm,
                              zero_offset=self.zero_offset, out_dtype=out_dtype)
+
+    def _strip_allowed(self) -> bool:
+        """Whether a strip copy may be made now, or none has to be."""
+        return self._strip_only or not _recording() or \
+            (self._strip is not None and self._strip_meta is not None and self._update())
 
     def _one_row_args(self) -> tuple | None:
         """``(strip copy, its scales and zeros, int16 gather index)`` of the strip GEMV, kept for

@@ -181,6 +181,50 @@ def test_changed_inside_a_capture(kernels, monkeypatch):
         assert all(torch.equal(lin(_x(m)), _linear(2, act)(_x(m))) for m in ROWS)
 
 
+@pytest.mark.parametrize("act", [False, True])
+@pytest.mark.parametrize("m", ROWS)
+def test_traced_before_any_call(kernels, act, m):
+    # a trace records torch's operations only: a copy that a kernel fills would be recorded as an
+    # uninitialised tensor, so none is made there and the buffers' own product is recorded
+    from torch.fx.experimental.proxy_tensor import make_fx
+    x, want = _x(m), _linear(1, act)(_x(m))
+    lin = _linear(1, act)
+    traced = torch.jit.trace(lin, x, check_trace=False)
+    assert lin._strip is None and lin._strip_meta is None
+    assert torch.equal(traced(x), want)
+    for pre in (False, True):
+        lin = _linear(1, act)
+        fx = make_fx(lambda t: lin(t), pre_dispatch=pre)(x)
+        assert lin._strip is None and torch.equal(fx(x), want)
+    lin = _linear(1, act)
+    rows = x.expand(2, m, K)
+    assert torch.equal(torch.func.vmap(lin)(rows)[1], want)
+    # the buffers of a linear that has run stay the traced graph's inputs for many rows
+    if m > 16:
+        lin(x)
+        traced = torch.jit.trace(lin, x, check_trace=False)
+        lin.scales.mul_(2)
+        assert torch.allclose(traced(x).float(), 2 * want.float(), rtol=1e-2)
+
+
+def test_traced_after_a_change(kernels):
+    # without act-order the buffers are read; with it the sorted weight would have to be made
+    # inside the trace (torch.jit.trace reads the module's properties first, which does it)
+    from torch.fx.experimental.proxy_tensor import make_fx
+    for act in (False, True):
+        for m in ROWS:
+            x, want = _x(m), _linear(2, act)(_x(m))
+            lin = _linear(1, act)
+            lin(x)
+            lin.load_state_dict(_linear(2, act).state_dict())
+            if act:
+                with pytest.raises(RuntimeError, match="or tracing"):
+                    make_fx(lambda t: lin(t))(x)
+            else:
+                assert torch.equal(make_fx(lambda t: lin(t))(x)(x), want)
+            assert torch.equal(torch.jit.trace(lin, x, check_trace=False)(x), want)
+
+
 def test_inference_tensors_are_read_at_every_call(kernels):
     # they keep no version, so a change in place leaves no mark: no copy of them is used for
     # the rows that were read from the buffers before there was one
