@@ -42,6 +42,18 @@ def _recording() -> bool:
         (_function_modes() > 0 and torch._ops._len_torch_dispatch_stack_pre_dispatch() > 0)
 
 
+def _capturing(t: torch.Tensor) -> bool:
+    """Whether a kernel on ``t`` would be captured into a graph: it then runs at replay only, and
+    what it writes lives in the graph's memory."""
+    return t.is_cuda and torch.cuda.is_current_stream_capturing()
+
+
+def _settle(t: torch.Tensor) -> None:
+    """Wait for a copy that was just made: the next call may read it on another stream."""
+    if t.is_cuda:
+        torch.cuda.current_stream(t.device).synchronize()
+
+
 def _stamp(buffers: dict) -> tuple:
     """What the copies made from a linear's buffers are valid for: each tensor with its version,
     which every in-place operation of torch counts up, and whether one of them keeps none (an
@@ -157,8 +169,7 @@ class GPTQLinear(torch.nn.Module):
         weight = not (same[0] and same[1]) and not self._strip_only and \
             (old is None or new[0].numel() > 0)
         recording = _recording()
-        if old is not None and (recording or new[4].is_cuda and
-                                torch.cuda.is_current_stream_capturing()):
+        if old is not None and (recording or _capturing(new[4])):
             if weight and self._perm is not None:
                 raise RuntimeError("the weight changed since its kernel copies were made: call "
                                    "post_init (or run the linear once) before capturing or "
@@ -184,6 +195,8 @@ class GPTQLinear(torch.nn.Module):
         if self._strip_meta is not None and not (same[2] and same[3]):
             sc, qz = ops.strip_meta(self.scales, self.qzeros, self.group_size)
             self._strip_meta = _into(self._strip_meta[0], sc), _into(self._strip_meta[1], qz)
+        if self._perm is not None or self._strip_meta is not None or self._strip is not None:
+            _settle(new[4])
         self._src = new
         return True
 
@@ -214,6 +227,9 @@ class GPTQLinear(torch.nn.Module):
         and ``reorder_output_columns`` raise ``RuntimeError``."""
         if self._strip_only:
             return self
+        if _capturing(self.scales):
+            raise RuntimeError("keep_strip_only frees the weight: not inside a graph capture, "
+                               "which fills the strip copy at replay only")
         self.stream_weight(strip=True)
         self.strip_meta()
         self._kernel_qweight = None
@@ -233,7 +249,8 @@ class GPTQLinear(torch.nn.Module):
         ``strip=False``: the wave-contiguous tiled copy of the kernel weight (split-K
         GEMV) when N % 64 == 0, else the kernel weight in row layout.  ``strip=True``:
         the column-strip copy for the full-K strip GEMV.  Copies are built once, and again
-        when the buffers change (:meth:`_update`)."""
+        when the buffers change (:meth:`_update`); one that is built inside a graph capture is
+        the caller's, for that capture only."""
         current = self._update()
         if strip and self._strip is not None and (current or self._strip_only):
             return self._strip, N.LAYOUT_STRIP
@@ -243,7 +260,8 @@ class GPTQLinear(torch.nn.Module):
                 raise RuntimeError(f"no strip layout for K={self.in_features}, "
                                    f"N={self.out_features}")
             copy = ops.strip_weights(qw)
-            if current:
+            if current and not _capturing(copy):
+                _settle(copy)
                 self._strip = copy
             return copy, N.LAYOUT_STRIP
         if self.out_features % 64:
@@ -251,38 +269,37 @@ class GPTQLinear(torch.nn.Module):
         if self._tiled is not None and current:
             return self._tiled, N.LAYOUT_TILED
         copy = ops.tile_weights(qw)
-        if current:
+        if current and not _capturing(copy):
+            _settle(copy)
             self._tiled = copy
         return copy, N.LAYOUT_TILED
 
     def strip_meta(self):
-        """``(scales, qzeros)`` in the strip order the strip GEMV reads (built once, and again
-        when either buffer changes)."""
+        """``(scales, qzeros)`` in the strip order the strip GEMV reads (kept as the copies of
+        :meth:`stream_weight`)."""
         current = self._update()
         if self._strip_meta is not None and current:
             return self._strip_meta
         meta = ops.strip_meta(self.scales, self.qzeros, self.group_size)
-        if current:
+        if current and not _capturing(meta[0]):
+            _settle(meta[0])
             self._strip_meta = meta
         return meta
 
     def _prompt_ready(self, x: torch.Tensor) -> bool:
         """Whether the prompt-length GEMM takes this linear's rows on the strip copy and its
-        metadata (made at the first such call, and waited for so that any stream may read them).
-        It does not where the AutoGPTQ buffers are read at every call and a copy would not follow
-        them: in a graph capture, a trace or compiled call or on a tensor subclass, and for
-        inference tensors, whose changes leave no mark."""
+        metadata (made at the first such call).  It does not where the AutoGPTQ buffers are read
+        at every call and a copy would not follow them: in a graph capture, a trace or compiled
+        call or on a tensor subclass, and for inference tensors, whose changes leave no mark."""
         if self.out_features % 128 or not x.is_cuda or _recording() or \
                 type(x) not in (torch.Tensor, torch.nn.Parameter) or self._src[8] or \
                 torch.cuda.is_current_stream_capturing():
             return False
         if self._strip is None or self._strip_meta is None:
-            scales = self._buffers["scales"]
-            if not self.supports_strip() or not scales.is_cuda:
+            if not self.supports_strip() or not self._buffers["scales"].is_cuda:
                 return False
             self.stream_weight(strip=True)
             self.strip_meta()
-            torch.cuda.current_stream(scales.device).synchronize()
         return True
 
     def drop_original(self) -> None:
@@ -323,11 +340,11 @@ class GPTQLinear(torch.nn.Module):
         through the act-order index while staging), few rows on the skinny strip GEMM where
         it pays (:func:`ops.strip_rows_pays`), more than 16 on the prompt-length GEMM (x
         gathered by a launch before it) where N is a multiple of 128; all read the strip copy
-        of the weight, built once and kept as long as the buffers stay as they are.  The others run on the split-K GEMM over the
-        AutoGPTQ layout, 16 rows at a time (4096 x 24576, g128, act-order: 33 us per 16 rows
-        against 30-70 us for 17 to 256 rows on the prompt-length GEMM).  Calls
-        go through the ``torch.ops.mtl`` operators (one dispatcher call, torch's stream and
-        allocator)."""
+        of the weight, built once and kept as long as the buffers stay as they are.  The others
+        run on the split-K GEMM over the AutoGPTQ layout, 16 rows at a time (4096 x 24576, g128,
+        act-order: 33 us per 16 rows against 30-70 us for 17 to 256 rows on the prompt-length
+        GEMM).  Calls go through the ``torch.ops.mtl`` operators (one dispatcher call, torch's
+        stream and allocator)."""
         m = x.numel() // self.in_features if self.in_features else 0
         current = self._update()
         if m == 1:
@@ -373,11 +390,13 @@ class GPTQLinear(torch.nn.Module):
             return None
         strip = self.stream_weight(strip=True)[0]
         sc, qz = self.strip_meta()
-        if perm is not None and self._perm16 is None:
-            self._perm16 = perm.to(torch.int16)
-        ready = strip, sc, qz, self._perm16
-        if strip is self._strip and sc is self._strip_meta[0]:
-            self._one_row = ready
+        perm16 = self._perm16
+        if perm is not None and perm16 is None:
+            perm16 = perm.to(torch.int16)
+        ready = strip, sc, qz, perm16
+        if strip is self._strip and not _recording() and not _capturing(strip) and self._update():
+            _settle(strip)
+            self._perm16, self._one_row = perm16, ready
         return ready
 
     def dequantize(self) -> torch.Tensor:

@@ -225,6 +225,41 @@ def test_traced_after_a_change(kernels):
             assert torch.equal(torch.jit.trace(lin, x, check_trace=False)(x), want)
 
 
+@pytest.mark.parametrize("act", [False, True])
+def test_first_call_inside_a_capture(kernels, monkeypatch, act):
+    # what a capture makes is filled at replay and lives in the graph's memory: it is used there
+    # and not kept, so an eager call before any replay reads copies of its own
+    for m in (1, 4):
+        lin, x = _linear(1, act), _x(m)
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+        lin(x)
+        assert all(c is None for c in (lin._strip, lin._strip_meta, lin._perm16, lin._one_row))
+        with pytest.raises(RuntimeError, match="capture"):
+            lin.keep_strip_only()
+        assert lin.qweight.numel()
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+        assert torch.equal(lin(_x(40)), _linear(1, act)(_x(40)))
+
+
+def test_copies_are_waited_for(kernels, monkeypatch):
+    # whichever call makes a copy, or makes it again, waits for it: the next may run on another
+    # stream
+    waits = []
+    stream = types.SimpleNamespace(synchronize=lambda: waits.append(1))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: stream)
+    for m in ROWS:
+        lin = _linear(1, True)
+        waits.clear()
+        lin(_x(m))
+        assert waits
+        waits.clear()
+        lin(_x(m))
+        assert not waits
+        lin.load_state_dict(_linear(2, True).state_dict())
+        lin(_x(m))
+        assert waits
+
+
 def test_inference_tensors_are_read_at_every_call(kernels):
     # they keep no version, so a change in place leaves no mark: no copy of them is used for
     # the rows that were read from the buffers before there was one
@@ -281,3 +316,33 @@ def test_buffers_changed_after_use_on_the_device(dev, act):
             # the captured many-row call runs on the AutoGPTQ layout: other fp32 sums, bf16 out
             err = (out.float() - want[m].float()).norm() / want[m].float().norm()
             assert torch.equal(out, want[m]) if m <= 16 else float(err) < 4e-3, (m, float(err))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", [False, True])
+@pytest.mark.parametrize("m", [1, 4])
+def test_first_call_captured_on_the_device(dev, act, m):
+    # a first call of one or few rows inside a capture, then an eager prompt before any replay,
+    # on another stream: both right, and every replay
+    def linear():
+        return gptq.GPTQLinear.from_buffers(*(None if b is None else b.to(dev)
+                                              for b in _buffers(1, act)), G).post_init()
+
+    x, x40 = _x(m).to(dev), _x(40).to(dev)
+    want, want40 = linear()(x), linear()(x40)
+    lin = linear()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = lin(x)
+    assert lin._strip is None
+    other = torch.cuda.Stream()
+    with torch.cuda.stream(other):
+        assert torch.equal(lin(x40), want40)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert torch.equal(lin(x), want) and torch.equal(lin(x40), want40)
