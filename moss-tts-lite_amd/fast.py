@@ -667,7 +667,7 @@ class FastDecoder:
         cfg, dev, bf = self.m.cfg, self.dev, torch.bfloat16
         z = lambda n, dt=bf: torch.zeros(rows, n, dtype=dt, device=dev)  # noqa: E731
         pf = {"rows": rows, "ids": z(self.table_ptrs.numel(), torch.int64), "h": z(cfg.hidden),
-              "x": z(cfg.hidden), "x_nat": z(cfg.hidden), "qkv": z(cfg.qkv_out),
+              "h_next": z(cfg.hidden), "x": z(cfg.hidden), "x_nat": z(cfg.hidden), "qkv": z(cfg.qkv_out),
               "q": z(cfg.n_heads * cfg.head_dim), "attn": z(cfg.hidden),
               "act": z(cfg.intermediate),
               "gate": z(cfg.intermediate) if any(self.up_keep) else None}
@@ -710,11 +710,11 @@ class FastDecoder:
             y.data_ptr(), ldy, pf["wide"].data_ptr(), pf["wide"].numel(), stream),
             "mtl_w4_gemm_prompt_qsz")
 
-    def _prefill_norm(self, rows: int, norm_w, nxt, out, stream) -> None:
+    def _prefill_norm(self, rows: int, h, norm_w, nxt, out, stream) -> None:
         """``out = RMSNorm(h)`` in the input order of ``nxt``, staged for its GEMM when that
         takes staged x."""
         cfg, pf, lib = self.m.cfg, self._pf, N.load()
-        args = (pf["h"].data_ptr(), cfg.hidden, norm_w.data_ptr(),
+        args = (h.data_ptr(), cfg.hidden, norm_w.data_ptr(),
                 None if nxt.perm is None else nxt.perm.data_ptr(), out.data_ptr(), cfg.hidden)
         if self._prefill_staged() and not self._wide_bytes(rows, nxt):
             N.check(lib.mtl_rmsnorm_gather_staged(*args, pf["xsum"].data_ptr(), rows, cfg.hidden,
@@ -793,7 +793,7 @@ class FastDecoder:
         if wide or not self.fuse_split_sums:
             gemm = self._prefill_wide if wide else self._prefill_gemm
             gemm(x_in, rows, lin, N.EPI_RESIDUAL, h, cfg.hidden, stream)
-            self._prefill_norm(rows, norm_w, nxt, out, stream)
+            self._prefill_norm(rows, h, norm_w, nxt, out, stream)
             return
         gather = nxt.perm
         staged = self._prefill_staged() and not self._wide_bytes(rows, nxt)
@@ -815,7 +815,8 @@ class FastDecoder:
         # Ids on the device are read back while the first launches (embedding, norm and GEMM,
         # into scratch buffers; ids outside a table read nothing) run, and checked before the
         # first K/V row is written (a 256-row layer: 231 -> 214 us, as the host queues the
-        # other launches without a gap).
+        # other launches without a gap).  The residual stream is one of two buffers: the rows
+        # that the prompt before returned outlive a refused one.
         host_ids = None
         if isinstance(ids, torch.Tensor) and ids.is_cuda and ids.device == self.h.device:
             host_ids = ids.to("cpu", non_blocking=True)
@@ -834,7 +835,8 @@ class FastDecoder:
         eps = ctypes.c_float(cfg.eps)
         scale = ctypes.c_float(attention_scale(cfg))
         p = lambda t: None if t is None else t.data_ptr()  # noqa: E731
-        h, x, qkv, q, attn, act = (pf[k] for k in ("h", "x", "qkv", "q", "attn", "act"))
+        h, x, qkv, q, attn, act = (pf[k] for k in ("h" if host_ids is None else "h_next", "x",
+                                                   "qkv", "q", "attn", "act"))
         H, Hkv, D = cfg.n_heads, cfg.n_kv_heads, cfg.head_dim
         N.check(lib.mtl_embed_rows(pf["ids"].data_ptr(), rows, self.table_ptrs.numel(),
                                    self.table_ptrs.data_ptr(), self.vocabs.data_ptr(), cfg.hidden,
@@ -843,7 +845,7 @@ class FastDecoder:
         for li, lyr in enumerate(m.layers):
             lq = lyr["qkv"]
             if li == 0:   # later layers' input norms ride on the previous down GEMM
-                self._prefill_norm(rows, lyr["input_layernorm"], lq, x, st)
+                self._prefill_norm(rows, h, lyr["input_layernorm"], lq, x, st)
             wide = self._wide_bytes(rows, lq)
             staged = self._prefill_staged() and not wide
             fuse_qkv = self.fuse_split_sums and not wide
@@ -857,6 +859,7 @@ class FastDecoder:
             if li == 0 and host_ids is not None:
                 read_back.synchronize()
                 _check_ids(host_ids, self.id_limits)
+                pf["h"], pf["h_next"] = h, pf["h"]
             if self.v_keep[li]:
                 # the bf16-kept v_proj (gptq.py:689-693) reads x in its natural order
                 x_v = x

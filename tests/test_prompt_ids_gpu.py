@@ -32,3 +32,27 @@ def test_refused_prompt_leaves_the_cache(dev, where):
         again.fill_(cfg.vocab + 5)
         torch.cuda.synchronize()
         assert torch.equal(h2, h)
+
+
+@pytest.mark.parametrize("where", ["device", "host"])
+def test_refused_prompt_leaves_the_returned_rows(dev, where):
+    # the rows of the last prompt are a view of a buffer: prompts refused after it, of any
+    # length, do not write into it, and the next accepted one is right
+    from moss_tts_lite_amd.fast import FastDecoder
+    from tests._decode_case import build_case, small_config
+    cfg = small_config()
+    model, _ = build_case(cfg, seed=4, dev=dev)
+    dec = FastDecoder(model)
+    ids = (torch.arange(20).reshape(-1, 1) * 7 % cfg.vocab).to(dev if where == "device" else "cpu")
+    other = (ids + 11) % cfg.vocab
+    want = [dec.prefill_rows(t).clone() for t in (ids, other)]
+    rows = dec.prefill_rows(ids)
+    for length in (20, 5, 20):
+        wrong = other[:length].clone()
+        wrong[length // 2, 0] = cfg.vocab
+        with pytest.raises(ValueError, match="outside its embedding table"):
+            dec.prefill_rows(wrong)
+        torch.cuda.synchronize()
+        assert torch.equal(rows, want[0])
+    assert torch.equal(dec.prefill_rows(other), want[1])
+    assert torch.equal(dec.prefill_rows(ids), want[0])
