@@ -158,9 +158,10 @@ int mtl_gptq_actorder_prepare(const int32_t* qweight, const int32_t* g_idx,
  *           (N*K/8 words; NOT torch's tiled bytes)
  *   qsz     bf16 [K/g, N, 2], read in place
  *   y       bf16 [M, N], 8-byte aligned
- *   workspace  NULL, or mtl_int4pack_mm_workspace_bytes(M, K, N) bytes: lets a launch
- *           with M > 1 split K over workgroups, or stage its operands (results then differ
- *           by fp32 rounding)
+ *   workspace  NULL, or mtl_int4pack_mm_group_workspace_bytes(M, K, N, g) bytes: lets a
+ *           launch with M > 1 split K over workgroups, or stage its operands (results then
+ *           differ by fp32 rounding); mtl_int4pack_mm_workspace_bytes is the most that any
+ *           group size takes
  * M = 1 runs the full-K strip GEMV (K <= 16384); 2 <= M <= 16 the skinny strip GEMM
  * (mtl_w4_gemm_strip_rows_ex), more rows the GEMM with dequantised operands
  * (mtl_w4_gemm_prompt_qsz) where it is the faster one and the workspace holds them, else the
@@ -168,6 +169,8 @@ int mtl_gptq_actorder_prepare(const int32_t* qweight, const int32_t* g_idx,
  * N % 16 == 0 (torch asks N % 8 only).
  */
 int64_t mtl_int4pack_mm_workspace_bytes(int64_t M, int64_t K, int64_t N);
+int64_t mtl_int4pack_mm_group_workspace_bytes(int64_t M, int64_t K, int64_t N,
+                                              int32_t group_size);
 int mtl_int4pack_mm(const void* x, int64_t M, int64_t K, const int32_t* packed,
                     int32_t group_size, const void* qsz, int64_t N, void* y,
                     void* workspace, int64_t ws_bytes, void* stream);

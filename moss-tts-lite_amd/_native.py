@@ -137,6 +137,7 @@ _SIGNATURES = {
                                       _i32, _i32, _i32, _c_void_p, _i64, _c_void_p, _i64,
                                       _c_void_p]),
     "mtl_int4pack_mm_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "mtl_int4pack_mm_group_workspace_bytes": (_i64, [_i64, _i64, _i64, _i32]),
     "mtl_embed_rows": (_i32, [_c_void_p, _i64, _i32, _c_void_p, _c_void_p, _i64, _c_void_p,
                               _c_void_p]),
     "mtl_rmsnorm_gather": (_i32, [_c_void_p, _i64, _c_void_p, _c_void_p, _c_void_p, _i64, _i64,

@@ -206,9 +206,9 @@ int strip_rows(const void* x, int64_t M, int64_t ldx, int64_t K, const int32_t* 
                int32_t out_dtype, void* stream);
 
 // The prompt-length GEMM on the reference's records with dequantised f16 operands
-// (mtl_w4wide.hip): whether it is the faster one for a shape (group 0: at any group size), the
-// workspace it needs (largest at group 32), and its launches.  Pointers, alignment and the
-// K % 256, N % 16 and K % group rules are checked by the caller.
+// (mtl_w4wide.hip): whether it is the faster one for a shape, the workspace it needs, and its
+// launches.  Pointers, alignment and the K % 256, N % 16 and K % group rules are checked by the
+// caller.
 int pf_device_cus();
 bool wide_pays(int64_t M, int64_t K, int64_t N, int32_t group);
 int64_t wide_workspace_bytes(int64_t M, int64_t K, int64_t N, int32_t group);

@@ -619,11 +619,7 @@ bool wide_pays(int64_t M, int64_t K, int64_t N, int32_t group) {
   if (cols / 16 * (K / 128) * 1024 >= ((int64_t)1 << 31) || cols * (K / 32) * 4 >= ((int64_t)1 << 31))
     return false;
   const int cus = pf_device_cus();
-  for (int32_t g = 32; g <= 256; g *= 2)
-    if ((group == 0 || g == group) && K % g == 0 &&
-        1.1 * wide_us(M, K, N, g, cus) < other_us(M, K, N, g, cus))
-      return true;
-  return false;
+  return 1.1 * wide_us(M, K, N, group, cus) < other_us(M, K, N, group, cus);
 }
 
 template <int MB, int KW>

@@ -55,7 +55,7 @@ at::Tensor weight_int4pack_mm(const at::Tensor& x, const at::Tensor& packed, int
   const int64_t M = x2.size(0);
   at::Tensor y = at::empty({M, N}, x2.options());
   if (M == 0) return y;
-  const int64_t ws = mtl_int4pack_mm_workspace_bytes(M, K, N);
+  const int64_t ws = mtl_int4pack_mm_group_workspace_bytes(M, K, N, (int32_t)g);
   at::Tensor wsb;
   if (ws > 0) wsb = at::empty({(ws + 3) / 4}, x2.options().dtype(at::kFloat));
   const hipStream_t stream = c10::hip::getCurrentHIPStream(x2.device().index()).stream();

@@ -38,6 +38,26 @@ def test_no_process_wide_tuning_state(lib):
     assert not hasattr(lib, "mtl_tune_set_strip_nb")
 
 
+def test_int4pack_workspace_is_that_of_the_route(lib):
+    # a call holds the staged operands of the GEMM with dequantised operands only where that runs
+    # it, at its own group size, and otherwise the prompt-length GEMM's split sums; the query
+    # without a group covers every group size
+    routes = set()
+    for m in (17, 64, 96, 128, 192, 256, 389, 1100, 1536):
+        for k, n in ((4096, 24576), (4096, 5120), (4096, 4096), (12288, 4096), (1024, 2000)):
+            split = lib.mtl_w4_gemm_prefill_workspace_bytes(m, k, n) if n % 128 == 0 else 0
+            need = {}
+            for g in (32, 64, 128, 256):
+                wide = lib.mtl_w4_gemm_prompt_qsz_workspace_bytes(m, k, n, g)
+                need[g] = lib.mtl_int4pack_mm_group_workspace_bytes(m, k, n, g)
+                assert need[g] == (wide or split), (m, k, n, g)
+                routes.add((g, wide > 0))
+            assert lib.mtl_int4pack_mm_workspace_bytes(m, k, n) == max(need.values())
+    assert len(routes) == 8
+    assert lib.mtl_int4pack_mm_group_workspace_bytes(256, 4096, 4096, 48) == 0
+    assert lib.mtl_int4pack_mm_group_workspace_bytes(1, 4096, 4096, 32) == 0
+
+
 def test_status_strings(lib):
     assert lib.mtl_status_string(0) == b"ok"
     assert lib.mtl_status_string(N.MTL_ERR_GROUP) == b"unsupported group size"
