@@ -205,3 +205,134 @@ def test_gptq_module_prompt_rows(dev, m, k, n, g, act):
         torch.cuda.synchronize()
         assert rel_l2(out.cpu().numpy(), case["y_ref"]) < TOL_F32
         assert torch.equal(fresh(x, out_dtype=torch.float32), y)
+
+
+def row_blocks(m, n, cus=256):
+    """(row tiles per workgroup, workgroups) as the launch chooses them: the rounds over the CUs
+    times the time of a turn at that many row tiles."""
+    tiles, ctiles, best, cost = -(-m // 16), -(-n // 256), 0, 0.0
+    for nb in range(-(-tiles // 6), tiles + 1):
+        rt = -(-tiles // nb)
+        c = -(-nb * ctiles // cus) * (2.3 if rt <= 4 else 2.7 if rt == 5 else 3.1)
+        if not best or c < cost:
+            best, cost = nb, c
+        if rt <= 4:
+            break
+    return -(-tiles // best), best * ctiles
+
+
+# every kernel instance: 4, 5 and 6 row tiles (at 3 and 4 also fewer than the instance holds), one
+# metadata record per block or two or four (g 128 / 256, 64, 32), K in halves or whole; K = 256
+# and 768 are one and three blocks of a half, two and six whole
+_INSTANCES = [(m, n, two, rt) for two, shapes in ((True, ((49, 256, 4), (80, 33024, 5), (89, 33040, 6))),
+                                                  (False, ((40, 98304, 4), (208, 33024, 5),
+                                                           (251, 33040, 6))))
+              for m, n, rt in shapes]
+
+
+@pytest.mark.parametrize("g", [32, 64, 128, 256])
+@pytest.mark.parametrize("m,n,two,rt", _INSTANCES)
+def test_prompt_gemm_every_instance(dev, m, n, two, rt, g):
+    tiles, groups = row_blocks(m, n)
+    assert max(tiles, 4) == rt and (2 * groups < 3 * 256) == two
+    for k in (256, 768) if n < 1000 else (256,):
+        packed, qsz, w = record(dev, n, k, g, m + g)
+        x = torch.randn(m, k, device=dev, generator=torch.Generator(device=dev).manual_seed(n)).bfloat16()
+        y = run(x, packed, qsz, g, N.EPI_NONE, torch.empty(m, n, device=dev))
+        ref = x.double() @ w.t()
+        assert rel(y, ref) < 2e-6
+        # each row tile and the last, ragged column tile by themselves
+        err = [float((a - b).norm() / b.norm()) for a, b in zip(y.double().split(16), ref.split(16))]
+        assert max(err) < 4e-6 and rel(y[:, n // 256 * 256 - 256:], ref[:, n // 256 * 256 - 256:]) < 4e-6
+        if n % 64 == 0:
+            act = run(x, packed, qsz, g, N.EPI_SILU_MUL,
+                      torch.empty(m, n // 2, device=dev, dtype=torch.bfloat16))
+            gu = y.bfloat16().float().reshape(m, n // 64, 2, 32)
+            want = torch.nn.functional.silu(gu[:, :, 0]).bfloat16().float() * gu[:, :, 1]
+            assert rel(act, want.reshape(m, -1).double()) < 2.5e-3
+        h = torch.randn(m, n, device=dev).bfloat16()
+        hr = (y.bfloat16().float() + h.float()).bfloat16()
+        assert torch.equal(run(x, packed, qsz, g, N.EPI_RESIDUAL, h), hr)
+
+
+def moss_backbone(dev, hidden, inter, g, max_seq, keep_up):
+    """Two layers of the reference's records with v_proj in bf16 and, with ``keep_up``, up_proj
+    of the first."""
+    from moss_tts_lite_amd import model
+    from moss_tts_lite_amd.gptq import QszLinear, interleave_qsz_gate_up
+    gen = torch.Generator(device=dev).manual_seed(hidden + inter)
+    heads, kv = hidden // 128, max(hidden // 512, 1)
+    randn = lambda *s, std=1.0: (torch.randn(*s, device=dev, generator=gen) * std).bfloat16()  # noqa: E731
+    norm = lambda n: (1 + 0.05 * torch.randn(n, device=dev, generator=gen)).bfloat16()  # noqa: E731
+
+    def lin(n, k, seed):
+        packed, qsz, _ = record(dev, n, k, g, seed)
+        return QszLinear(packed, qsz, g)
+
+    layers = []
+    for i in range(2):
+        lw = {"input_layernorm": norm(hidden), "post_attention_layernorm": norm(hidden),
+              "q_norm": norm(128), "k_norm": norm(128), "qkv": lin((heads + kv) * 128, hidden, 10 * i),
+              "v": randn(kv * 128, hidden, std=0.02), "o": lin(hidden, hidden, 10 * i + 1),
+              "down": lin(hidden, inter, 10 * i + 2)}
+        gate, up = lin(inter, hidden, 10 * i + 3), lin(inter, hidden, 10 * i + 4)
+        if keep_up and i == 0:
+            lw.update(gate=gate, up=randn(inter, hidden, std=0.02))
+        else:
+            lw["gate_up"] = interleave_qsz_gate_up(gate, up)
+        layers.append(lw)
+    cfg = model.BackboneConfig(hidden=hidden, n_heads=heads, n_kv_heads=kv, head_dim=128,
+                               intermediate=inter, n_layers=2, vocab=64, group_size=g,
+                               act_order=False, max_seq=max_seq, n_vq=2, audio_vocab=33,
+                               audio_pad_code=32, two_way_ids=(0, 1))
+    return model.Int4Backbone(cfg, {
+        "layers": layers, "embed_tokens": randn(64, hidden), "final_norm": norm(hidden),
+        "head": randn(64, hidden, std=0.02), "emb_ext": list(randn(2, 33, hidden, std=0.2)),
+        "head_audio": randn(2, 33, hidden, std=0.02)})
+
+
+# the full width at a length where every linear takes this GEMM by itself, and small layers where
+# it is made to: all of them, and each alone (plain x into one GEMM, staged x into the next)
+@pytest.mark.parametrize("hidden,inter,rows,only", [
+    (4096, 12288, 1100, "rule"), (512, 1024, 70, "all"), (512, 1024, 70, "qkv"),
+    (512, 1024, 70, "o"), (512, 1024, 70, "gate_up"), (512, 1024, 70, "down")])
+@pytest.mark.parametrize("keep_up", [False, True])
+def test_prompt_layers_on_this_gemm(dev, monkeypatch, hidden, inter, rows, only, keep_up):
+    # kept v_proj on plain x, the residual into h before the next norm, SiLU*up, the last layer's
+    # down, kept up_proj: against the same layers on the prompt-length GEMM
+    from moss_tts_lite_amd.fast import FastMossDecoder
+    model = moss_backbone(dev, hidden, inter, 32, rows + 8, keep_up)
+    dec = FastMossDecoder(model)
+    gen = torch.Generator(device=dev).manual_seed(rows)
+    ids = torch.stack([torch.randint(0, n, (rows,), device=dev, generator=gen)
+                       for n in (64, 33, 33)], 1)
+    names = {id(lyr[k]): k for lyr in model.layers for k in ("qkv", "o", "gate_up", "down")}
+    asked = set()
+
+    def wide_bytes(self, m, lin):
+        if only not in ("all", names[id(lin)]):
+            return 0
+        asked.add(names[id(lin)])
+        return workspace(m, lin.in_features, lin.out_features, lin.group_size, "meta").numel()
+
+    def prompt():
+        model.reset_cache()
+        h = dec.prefill_rows(ids).clone()
+        return h, model.k_cache[:, :, :rows].clone(), model.v_cache[:, :, :rows].clone()
+
+    if only == "rule":
+        dec._prefill_io(rows)
+        assert all(dec._wide_bytes(rows, lyr[k]) for lyr in model.layers
+                   for k in ("qkv", "o", "gate_up", "down") if not (keep_up and k == "gate_up"))
+    else:
+        monkeypatch.setattr(FastMossDecoder, "_wide_bytes", wide_bytes)
+    got = prompt()
+    assert only == "rule" or asked == ({only} if only != "all" else {"qkv", "o", "gate_up", "down"})
+    monkeypatch.setattr(FastMossDecoder, "_wide_bytes", lambda self, m, lin: 0)
+    want = prompt()
+    # the two differ by fp32 rounding before each of about seven bf16 roundings a layer (2^-9 /
+    # sqrt(3) where one flips): below sqrt(2 * 7 * 2) * 1.1e-3 = 6e-3 over two layers
+    for a, b in zip(got, want):
+        assert torch.isfinite(a).all() and rel(a.float(), b.double()) < 6e-3
+    # layer 0's value rows come from the bf16 v_proj on the same normed rows
+    assert torch.equal(got[2][0], want[2][0])
