@@ -134,12 +134,6 @@ __device__ __forceinline__ float slot_total(const float* slots, int n, int lane)
 __device__ __forceinline__ float lo_bf(uint32_t w) { return bf16_to_f32(w & 0xffffu); }
 __device__ __forceinline__ float hi_bf(uint32_t w) { return bf16_to_f32(w >> 16); }
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-  return v;
-}
-
 // The same cross-lane steps on the VALU, for code where all 64 lanes are active: a
 // __shfl_xor is a ds_bpermute, an LDS round trip of about 85 cycles that the next step
 // waits for; these are a few cycles each.  xor 32 and xor 16 come from v_permlane32_swap /
@@ -147,10 +141,9 @@ __device__ __forceinline__ float wave_max(float v) {
 // x[i ^ 16] in some order, and addition and max are commutative); xor 8 and xor 4 are DPP
 // row rotations, which equal them once the values depend only on the lane modulo 16 and 8
 // (true after the larger steps of a butterfly that goes 32, 16, 8, 4, 2, 1); xor 2 and 1
-// are DPP quad permutations.  So wave_sum_valu / wave_max_valu give the bits of wave_sum /
-// wave_max.  The swaps are inline asm with both registers in and out (the compiler's
-// builtin loses the second result when both inputs are the same value), with the wait
-// states around them explicit.
+// are DPP quad permutations.  So wave_sum_valu gives the bits of wave_sum.  The swaps are
+// inline asm with both registers in and out (the compiler's builtin loses the second result
+// when both inputs are the same value), with the wait states around them explicit.
 __device__ __forceinline__ void permlane_swap16(uint32_t& a, uint32_t& b) {
   asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
 }

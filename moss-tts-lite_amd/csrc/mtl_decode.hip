@@ -405,8 +405,7 @@ struct AttnArgs {
 
 // The merge of one kv head's chunk partials (m, l, o[128]) per q head, in chunk order,
 // by the last workgroup of that kv head to finish; out[h*128 + d] (through out_index).
-// VALU: the wave reductions on the VALU (wave_max_valu, wave_sum_valu; the same bits).
-template <bool VALU, bool LOCAL = false>
+template <bool LOCAL>
 __device__ __forceinline__ void attn_merge(const AttnArgs& a, int kvh, int nch, int n_rep,
                                            int wave, int lane, float (*w_lds)[kAttnMaxChunks]) {
   // LOCAL: the partials were written by workgroups of this XCD and sit in its L2; the
@@ -457,11 +456,10 @@ __device__ __forceinline__ void attn_merge(const AttnArgs& a, int kvh, int nch, 
     };
     load_batch(0);
     {
-      const float M = VALU ? wave_max_valu(lc > 0.f ? mc : -INFINITY)
-                           : wave_max(lc > 0.f ? mc : -INFINITY);
+      const float M = wave_max_valu(lc > 0.f ? mc : -INFINITY);
       const float wc = lc > 0.f ? expf(mc - M) : 0.f;
       w_lds[wave][lane] = wc;
-      lc = VALU ? wave_sum_valu(wc * lc) : wave_sum(wc * lc);   // Ls from here on
+      lc = wave_sum_valu(wc * lc);                   // Ls from here on
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -799,7 +797,7 @@ __global__ void __launch_bounds__(256) attn_tile_kernel(AttnArgs a) {
     }
     __syncthreads();
     if (!last_flag) return;
-    attn_merge<true, true>(a, kvh, nch, n_rep, wave, lane, w_lds);
+    attn_merge<true>(a, kvh, nch, n_rep, wave, lane, w_lds);
     return;
   }
   // Agent-scope hand-off.  The count is a release (every partial store of the workgroup happens
@@ -815,7 +813,7 @@ __global__ void __launch_bounds__(256) attn_tile_kernel(AttnArgs a) {
   if (!last_flag) return;
   if (t == 0)
     __hip_atomic_store(&a.counters[kvh], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  attn_merge<true>(a, kvh, nch, n_rep, wave, lane, w_lds);
+  attn_merge<false>(a, kvh, nch, n_rep, wave, lane, w_lds);
 }
 
 // ----------------------------------------------------------------------------------
