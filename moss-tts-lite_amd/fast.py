@@ -714,8 +714,9 @@ class FastDecoder:
         """``out = RMSNorm(h)`` in the input order of ``nxt``, staged for its GEMM when that
         takes staged x."""
         cfg, pf, lib = self.m.cfg, self._pf, N.load()
+        perm = nxt.perm
         args = (h.data_ptr(), cfg.hidden, norm_w.data_ptr(),
-                None if nxt.perm is None else nxt.perm.data_ptr(), out.data_ptr(), cfg.hidden)
+                None if perm is None else perm.data_ptr(), out.data_ptr(), cfg.hidden)
         if self._prefill_staged() and not self._wide_bytes(rows, nxt):
             N.check(lib.mtl_rmsnorm_gather_staged(*args, pf["xsum"].data_ptr(), rows, cfg.hidden,
                                                   ctypes.c_float(cfg.eps), stream),
@@ -727,8 +728,7 @@ class FastDecoder:
     def _prefill_gemm(self, x, rows: int, lin, epilogue: int, y, ldy: int, stream) -> None:
         """One prompt-length int4 GEMM on the strip copy of ``lin`` (mtl_w4_gemm_prefill,
         or mtl_w4_gemm_prefill_qsz for the reference's records)."""
-        qw, layout = lin.stream_weight(True)
-        sc, qz = lin.strip_meta()
+        qw, layout, sc, qz = lin.strip_args()
         ws = ops.prefill_workspace(self.dev, rows, lin.in_features, lin.out_features)
         if layout == N.LAYOUT_STRIP_QSZ:
             N.check(N.load().mtl_w4_gemm_prefill_qsz(
@@ -751,8 +751,7 @@ class FastDecoder:
     def _prefill_gemm_staged(self, x, xsum, rows: int, lin, epilogue: int, y, ldy: int,
                              stream) -> None:
         """One prompt-length int4 GEMM on staged x (mtl_w4_gemm_prefill_staged)."""
-        qw, layout = lin.stream_weight(True)
-        sc, qz = lin.strip_meta()
+        qw, layout, sc, qz = lin.strip_args()
         qsz = layout == N.LAYOUT_STRIP_QSZ
         ws = ops.prefill_workspace(self.dev, rows, lin.in_features, lin.out_features)
         N.check(N.load().mtl_w4_gemm_prefill_staged(
@@ -769,8 +768,7 @@ class FastDecoder:
         launch that sums them (mtl_qk_norm_rope_kv_rows_partials,
         mtl_residual_rmsnorm_gather)."""
         lib = N.load()
-        qw, layout = lin.stream_weight(True)
-        sc, qz = lin.strip_meta()
+        qw, layout, sc, qz = lin.strip_args()
         qsz = layout == N.LAYOUT_STRIP_QSZ
         K, Nc = lin.in_features, lin.out_features
         N.check(lib.mtl_w4_gemm_prefill_partials(
@@ -814,9 +812,10 @@ class FastDecoder:
         m, cfg = self.m, self.m.cfg
         # Ids on the device are read back while the first launches (embedding, norm and GEMM,
         # into scratch buffers; ids outside a table read nothing) run, and checked before the
-        # first K/V row is written (a 256-row layer: 231 -> 214 us, as the host queues the
-        # other launches without a gap).  The residual stream is one of two buffers: the rows
-        # that the prompt before returned outlive a refused one.
+        # first K/V row is written: the host queues the other launches without a gap (one layer
+        # among others, 256 rows 232 -> 207 us, 60 rows 139 -> 118; alone no faster).  The
+        # residual stream is one of two buffers: the rows that the prompt before returned
+        # outlive a refused one.
         host_ids = None
         if isinstance(ids, torch.Tensor) and ids.is_cuda and ids.device == self.h.device:
             host_ids = ids.to("cpu", non_blocking=True)

@@ -215,7 +215,8 @@ class GPTQLinear(torch.nn.Module):
     def perm(self) -> torch.Tensor | None:
         """The act-order gather index (int32 ``[K]``: sorted row i is input channel
         ``perm[i]``), or None when the groups are contiguous."""
-        self._update()
+        if not self._strip_only:
+            self._update()
         return self._perm
 
     @torch.no_grad()
@@ -285,6 +286,15 @@ class GPTQLinear(torch.nn.Module):
             _settle(meta[0])
             self._strip_meta = meta
         return meta
+
+    def strip_args(self) -> tuple:
+        """``(weight, layout, metadata, zeros)`` of the strip kernels for a decoder, whose launches
+        hold the copies' addresses for as long as it lives: the copies as they are (made if they
+        are not there), without the look at the buffers that :meth:`forward` takes at each call
+        (0.8 us on the host, in a prompt at every linear of every layer)."""
+        if self._strip is None or self._strip_meta is None:
+            return self.stream_weight(strip=True) + self.strip_meta()
+        return (self._strip, N.LAYOUT_STRIP) + self._strip_meta
 
     def _prompt_ready(self, x: torch.Tensor) -> bool:
         """Whether the prompt-length GEMM takes this linear's rows on the strip copy and its
@@ -451,6 +461,10 @@ class QszLinear:
     def strip_meta(self):
         """``(metadata, zeros)`` in the strip kernels' argument order: qsz, none."""
         return self.qsz, None
+
+    def strip_args(self) -> tuple:
+        """``(weight, layout, metadata, zeros)`` in one, as GPTQLinear's."""
+        return self.packed, N.LAYOUT_STRIP_QSZ, self.qsz, None
 
     perm = None          # contiguous groups: no act-order gather
 

@@ -124,6 +124,18 @@ def test_copies_are_made_again_in_place(kernels):
     assert lin._strip is made
 
 
+def test_a_decoder_reads_the_copies_as_they_are(kernels):
+    # made at the first request, at the same addresses after a change that a call has followed
+    lin = _linear(1, True)
+    args = lin.strip_args()
+    assert args == lin.stream_weight(True) + lin.strip_meta()
+    lin.load_state_dict(_linear(2, True).state_dict())
+    assert lin.strip_args()[0] is args[0] and torch.equal(args[0], _linear(1, True).strip_args()[0])
+    lin(_x(40))
+    new = _linear(2, True).strip_args()
+    assert all(torch.equal(args[i], new[i]) for i in (0, 2, 3)) and lin.strip_args()[0] is args[0]
+
+
 def test_dropped_and_reordered_weights_keep_their_copies(kernels):
     # after drop_original or keep_strip_only the copies are all there is of the weight; the
     # metadata still follows its buffers
