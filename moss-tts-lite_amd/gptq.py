@@ -228,11 +228,10 @@ class GPTQLinear(torch.nn.Module):
         and ``reorder_output_columns`` raise ``RuntimeError``."""
         if self._strip_only:
             return self
-        if _capturing(self.scales):
+        if _capturing(self.scales) or _recording():
             raise RuntimeError("keep_strip_only frees the weight: not inside a graph capture, "
-                               "which fills the strip copy at replay only")
-        self.stream_weight(strip=True)
-        self.strip_meta()
+                               "which fills the strip copy at replay only, nor inside a trace")
+        self._copies("_strip", "_strip_meta")
         self._kernel_qweight = None
         self._tiled = None
         self.qweight = torch.empty(0, dtype=torch.int32, device=self.scales.device)
@@ -252,49 +251,54 @@ class GPTQLinear(torch.nn.Module):
         the column-strip copy for the full-K strip GEMV.  Copies are built once, and again
         when the buffers change (:meth:`_update`); one that is built inside a graph capture is
         the caller's, for that capture only."""
-        current = self._update()
-        if strip and self._strip is not None and (current or self._strip_only):
-            return self._strip, N.LAYOUT_STRIP
-        qw = self.kernel_args()[0]
         if strip:
-            if not self.supports_strip():
-                raise RuntimeError(f"no strip layout for K={self.in_features}, "
-                                   f"N={self.out_features}")
-            copy = ops.strip_weights(qw)
-            if current and not _capturing(copy):
-                _settle(copy)
-                self._strip = copy
-            return copy, N.LAYOUT_STRIP
+            return self._copies("_strip")[0], N.LAYOUT_STRIP
         if self.out_features % 64:
-            return qw, N.LAYOUT_ROWS
-        if self._tiled is not None and current:
-            return self._tiled, N.LAYOUT_TILED
-        copy = ops.tile_weights(qw)
-        if current and not _capturing(copy):
-            _settle(copy)
-            self._tiled = copy
-        return copy, N.LAYOUT_TILED
+            return self.kernel_args()[0], N.LAYOUT_ROWS
+        return self._copies("_tiled")[0], N.LAYOUT_TILED
 
     def strip_meta(self):
         """``(scales, qzeros)`` in the strip order the strip GEMV reads (kept as the copies of
         :meth:`stream_weight`)."""
+        return self._copies("_strip_meta")[0]
+
+    def _copies(self, *names: str) -> list:
+        """The copies ``names`` (attributes), made where they are not there.  New ones are kept,
+        after one wait for all of them, except where a capture fills them or a trace records
+        them."""
         current = self._update()
-        if self._strip_meta is not None and current:
-            return self._strip_meta
-        meta = ops.strip_meta(self.scales, self.qzeros, self.group_size)
-        if current and not _capturing(meta[0]):
-            _settle(meta[0])
-            self._strip_meta = meta
-        return meta
+        out = [getattr(self, n) if current or (n == "_strip" and self._strip_only) else None
+               for n in names]
+        missing = [i for i, c in enumerate(out) if c is None]
+        for i in missing:
+            out[i] = self._copy(names[i])
+        if missing and current and not _recording() and not _capturing(self._buffers["scales"]):
+            _settle(self._buffers["scales"])
+            for i in missing:
+                setattr(self, names[i], out[i])
+        return out
+
+    def _copy(self, name: str):
+        if name == "_strip_meta":
+            return ops.strip_meta(self.scales, self.qzeros, self.group_size)
+        if name == "_perm16":
+            return self._perm.to(torch.int16)
+        qw = self.kernel_args()[0]
+        if name == "_tiled":
+            return ops.tile_weights(qw)
+        if not self.supports_strip():
+            raise RuntimeError(f"no strip layout for K={self.in_features}, N={self.out_features}")
+        return ops.strip_weights(qw)
 
     def strip_args(self) -> tuple:
         """``(weight, layout, metadata, zeros)`` of the strip kernels for a decoder, whose launches
         hold the copies' addresses for as long as it lives: the copies as they are (made if they
         are not there), without the look at the buffers that :meth:`forward` takes at each call
         (0.8 us on the host, in a prompt at every linear of every layer)."""
-        if self._strip is None or self._strip_meta is None:
-            return self.stream_weight(strip=True) + self.strip_meta()
-        return (self._strip, N.LAYOUT_STRIP) + self._strip_meta
+        strip, meta = self._strip, self._strip_meta
+        if strip is None or meta is None:
+            strip, meta = self._copies("_strip", "_strip_meta")
+        return (strip, N.LAYOUT_STRIP) + meta
 
     def _prompt_ready(self, x: torch.Tensor) -> bool:
         """Whether the prompt-length GEMM takes this linear's rows on the strip copy and its
@@ -308,8 +312,7 @@ class GPTQLinear(torch.nn.Module):
         if self._strip is None or self._strip_meta is None:
             if not self.supports_strip() or not self._buffers["scales"].is_cuda:
                 return False
-            self.stream_weight(strip=True)
-            self.strip_meta()
+            self._copies("_strip", "_strip_meta")
         return True
 
     def drop_original(self) -> None:
@@ -398,15 +401,13 @@ class GPTQLinear(torch.nn.Module):
         perm = self._perm
         if not self.supports_strip() or (perm is not None and self.in_features > 12288):
             return None
-        strip = self.stream_weight(strip=True)[0]
-        sc, qz = self.strip_meta()
-        perm16 = self._perm16
-        if perm is not None and perm16 is None:
-            perm16 = perm.to(torch.int16)
-        ready = strip, sc, qz, perm16
-        if strip is self._strip and not _recording() and not _capturing(strip) and self._update():
-            _settle(strip)
-            self._perm16, self._one_row = perm16, ready
+        if perm is None:
+            (strip, meta), perm16 = self._copies("_strip", "_strip_meta"), None
+        else:
+            strip, meta, perm16 = self._copies("_strip", "_strip_meta", "_perm16")
+        ready = strip, meta[0], meta[1], perm16
+        if strip is self._strip and meta is self._strip_meta and perm16 is self._perm16:
+            self._one_row = ready
         return ready
 
     def dequantize(self) -> torch.Tensor:
