@@ -12,17 +12,19 @@
 // MFMA contraction over 3 K / g (9 % of the main one at g = 32, 2 % at 128).
 //
 // Measured, both launches, against mtl_w4prefill.hip on one chip: 389 x 4096 x 24576 at g = 32
-// 171 -> 96 us (815 TFLOP/s), 1100 x 4096 x 24576 at g = 32 401 -> 249 us, 1536 x 12288 x 4096
-// at g = 128 193 -> 155 us (995 TFLOP/s; a large bf16 matrix product of the library reaches
+// 173 -> 98 us (800 TFLOP/s), 1100 x 4096 x 24576 at g = 32 404 -> 253 us, 1536 x 12288 x 4096
+// at g = 128 195 -> 157 us (985 TFLOP/s; a large bf16 matrix product of the library reaches
 // 1450 here).
 //
 // Range.  A launch before the GEMM (wide_stage_kernel) finds a power of two per row of x and
 // per column of W that puts the largest magnitude of x at 2^6 .. 2^7 and of 8 s and z at
 // 2^13 .. 2^14; the result is scaled back exactly.  A bf16 x within 2^23 of its row's maximum
-// and a scale or zero within 2^23 of its column's are then exact in f16; smaller ones keep an
-// absolute error of 2^-25 (x: 2^-31 of the row's maximum, s and z: 2^-38 of the column's),
-// under the rounding of the fp32 sums.  X, the fp32 sum of a group's x, enters as three f16
-// parts.
+// and a scale or zero within 2^23 of its column's are then exact in f16; smaller ones are cut
+// (towards zero) with an absolute error below 2^-24 (x: 2^-30 of the row's maximum, s and z:
+// 2^-37 of the column's), under the rounding of the fp32 sums.  X, the fp32 sum of a group's x,
+// enters as three f16 parts.  fp32 output against float64, this GEMM and mtl_w4prefill.hip:
+// 2.6e-7 and 8.7e-7 at 389 x 4096 x 4096, g = 32, and with one channel in 256 at 2^10 to 2^26
+// times the others 3.3e-7 at most and 1.6e-6 to 3e-6.
 #include "mtl_w4core.h"
 #include "mtl_w4wide_reads.h"
 
@@ -237,21 +239,6 @@ __device__ __forceinline__ void dequant_step(uint32_t w, u32x4& t, uint32_t lo, 
   asm volatile("" : "+v"(t.x), "+v"(t.y), "+v"(t.z), "+v"(t.w));   // keeps the step here
 }
 
-// A workgroup owns RT row tiles x 256 columns; wave (kg, wn) multiplies all RT tiles by 64
-// columns (4 strips) over part kg of the K blocks.  Either way two waves share a SIMD: KW = 2 is
-// a workgroup of 8 waves per CU whose two halves of K meet in LDS at the end, for grids that
-// would not give every CU two workgroups; KW = 1 two independent workgroups of 4 waves, whose
-// barriers do not hold each other up (1100 x 4096 x 24576: 308 -> 289 us at g = 32, 265 -> 235
-// at g = 128; 389 rows 129 -> 119; but 1100 x 12288 x 4096, 224 workgroups: 159 -> 200).  RT = 6 is what three x buffers leave of the LDS: a
-// dequantised operand (12 VALU instructions per 8 codes) feeds 6 MFMAs and an x operand 4.
-// The x tiles come by direct loads into LDS two turns ahead (the staged order is the operand
-// order, so there is no conversion and no bank conflict), weights and scales into registers
-// three turns ahead.
-//
-// What bounds it at 1536 x 12288 x 4096, g = 128 (counters: 1.97 GHz, MFMA busy 53 % of the
-// cycles, LDS 13 %): the instructions a wave issues.  A turn (128 channels per wave) takes 2.0 us
-// at RT = 4; 1.2 with the dequantisation left out, 1.2 with the MFMAs left out, and 1.9 without
-// the x loads.  Two buffers instead of three and weights one turn ahead cost 5 %.
 // Four bf16 results of one row, as one store where rows and base allow it.
 __device__ __forceinline__ void put4(uint16_t* p, const uint32_t (&o)[4], int pack) {
   if (pack) {
@@ -276,6 +263,23 @@ __device__ __forceinline__ void wait_and_barrier() {
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
+// A workgroup owns RT row tiles x 256 columns; wave (kg, wn) multiplies all RT tiles by 64
+// columns (4 strips) over part kg of the K blocks.  Either way two waves share a SIMD: KW = 2 is
+// a workgroup of 8 waves per CU whose two halves of K meet in LDS at the end, for grids that
+// would not give most CUs two workgroups; KW = 1 two independent workgroups of 4 waves, whose
+// barriers do not hold each other up.  Halves against whole K, both launches: 1100 x 4096 x 24576
+// 282 / 254 us at g = 32 and 251 / 226 at g = 128, 389 rows at g = 32 108 / 101; but
+// 1100 x 12288 x 4096 at g = 32, 224 workgroups, 143 / 175.  RT = 6 is what three x buffers leave
+// of the LDS: a dequantised operand (12 VALU instructions per 8 codes) feeds 6 MFMAs and an x
+// operand 4.  The x tiles come by direct loads into LDS two turns ahead (the staged order is the
+// operand order, so there is no conversion and no bank conflict), weights and scales into
+// registers three turns ahead.
+//
+// What bounds it at 1536 x 12288 x 4096, g = 128 (counters of an earlier build of this tile,
+// 143 us: 1.97 GHz, MFMA busy 53 % of the cycles, LDS 13 %): the instructions a wave issues.  A
+// turn (128 channels per wave) took 2.0 us at RT = 4; 1.2 with the dequantisation left out, 1.2
+// with the MFMAs left out, and 1.9 without the x loads.  Two buffers instead of three and weights
+// one turn ahead cost 5 %.
 template <int RT, int MB, int KW>
 __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 w4_wide_kernel(WideArgs a) {
@@ -604,14 +608,19 @@ static double other_us(int64_t M, int64_t K, int64_t N, int32_t group, int cus) 
          (split > 0 ? 4.0 + split : 0.0);
 }
 
-// Measured (us, this GEMM against the other, both launches of each; 256 CUs):
-//   K x N, g          M = 96        192          389           600            1100
-//   4096 x 24576, 32  49 / 55     60 / 89      99 / 172     143 / 230      249 / 401
-//   4096 x 24576, 128 40 / 41     51 / 66      85 / 123     126 / 165      221 / 284
-//   12288 x 4096, 32 105 / 33    108 / 44     114 / 97      117 / 128      140 / 221
-//   4096 x 4096, 128  38 / 18     40 / 23      44 / 34       45 / 40        52 / 64
-//   1024 x 2000, 32   19 / 29     20 / 58      21 / 121      22 / 185       24 / 337
-// so the line lies where the estimates cross, with a tenth in hand, from 64 rows on.
+// Measured (us, this GEMM / the other, both launches of each, 256 CUs; * where the rule takes it):
+//   K x N, g          M = 96     128      192      256      389       600       1100
+//   4096 x 24576, 32  48 / 55    48/58*   59/87*   81/96    98/173*   145/234*  253/404*
+//   4096 x 24576, 128 40 / 41    41/45*   52/67*   70/69    87/123*   129/167*  226/290*
+//   12288 x 4096, 32  106 / 35   107/37   109/47   110/58   110/99    113/131   142/227*
+//   12288 x 4096, 128 90 / 28    92/29    93/36    94/43    94/74     96/97     128/163*
+//   4096 x 4096, 128  37 / 19    38/21    39/23    40/24    41/34     43/40     53/65*
+//   4096 x 5120, 32   43 / 25    45/27    46/29    47/35    47/51     48/71*    66/102*
+//   1024 x 2000, 32   19 / 29*   20/39*   20/59*   21/78*   21/121*   22/185*   25/337*
+// The line lies where the estimates cross, with a tenth in hand, from 64 rows on.  wide_us counts
+// one workgroup per CU in a round, also for the grids that run two (KW = 1), so it errs towards
+// the other GEMM: 96 and 256 rows of 4096 x 24576 at g = 32 and 600 of 12288 x 4096 stay there,
+// 7 to 18 us slower than here.  No shape of a sweep over 64 to 1536 rows was found slower here.
 bool wide_pays(int64_t M, int64_t K, int64_t N, int32_t group) {
   if (M < 64 || M > (1 << 20) || K < 256 || K % 256 != 0 || K > 65536 || N < 16 || N % 16 != 0)
     return false;
