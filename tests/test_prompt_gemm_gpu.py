@@ -336,3 +336,37 @@ def test_prompt_layers_on_this_gemm(dev, monkeypatch, hidden, inter, rows, only,
         assert torch.isfinite(a).all() and rel(a.float(), b.double()) < 6e-3
     # layer 0's value rows come from the bf16 v_proj on the same normed rows
     assert torch.equal(got[2][0], want[2][0])
+
+
+@pytest.mark.parametrize("zero_offset", [0, 1])
+@pytest.mark.parametrize("act", [True, False])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_gptq_module_route_against_split_k(dev, zero_offset, act, dt):
+    # the new route of many rows against the split-K GEMM over what a module takes: both zero
+    # conventions and output types, x 2 bytes off a 16-byte boundary, transposed, expanded, with
+    # leading dimensions, the row counts around 16, a tile and two of them
+    from moss_tts_lite_amd.gptq import GPTQLinear
+    from oracle import synth
+    from tests.test_gemm_gpu import t_bf16, t_f16, t_i32
+
+    k, n, g = 768, 256, 64
+    case = synth.gptq_case(k=k, n=n, m=130, group=g, act_order=act, seed=31 + zero_offset)
+    lin = GPTQLinear.from_buffers(t_i32(case["qweight"], dev), t_i32(case["qzeros"], dev),
+                                  t_f16(case["scales"], dev),
+                                  t_i32(case["g_idx"], dev) if act else None, g,
+                                  zero_offset=zero_offset).post_init()
+    x = t_bf16(case["x_bits"], dev)
+    w = lin.dequantize().double()
+    off = torch.cat([x.new_zeros(1), x.reshape(-1)])[1:].reshape(130, k)
+    forms = [x[:m] for m in (15, 16, 17, 63, 64, 65, 130)]
+    forms += [off, x[:64].t().contiguous().t(), x[:1].expand(40, k), x[:120].reshape(2, 3, 20, k)]
+    qw, qz, sc, perm = lin.kernel_args()
+    for xf in forms:
+        y = lin(xf, out_dtype=dt)
+        old = ops.gptq_gemm(xf.clone(memory_format=torch.contiguous_format), qw, qz, sc, g,
+                            perm=perm, zero_offset=zero_offset, out_dtype=dt)
+        ref = xf.double() @ w
+        assert y.shape == old.shape == ref.shape and y.dtype == dt
+        # 32-bit sums in another order, or those rounded to bf16 (2^-9 / sqrt(3) of each value)
+        bar = 4e-6 if dt == torch.float32 else 2.5e-3
+        assert rel(y, ref) < bar and rel(y, ref) < 2 * rel(old, ref) + 1e-7
