@@ -57,7 +57,8 @@ def _settle(t: torch.Tensor) -> None:
 def _stamp(buffers: dict) -> tuple:
     """What the copies made from a linear's buffers are valid for: each tensor with its version,
     which every in-place operation of torch counts up, and whether one of them keeps none (an
-    inference tensor)."""
+    inference tensor).  A write that torch does not count (a collective into a buffer, ``.data``,
+    a raw pointer) leaves no mark: ``post_init`` makes the copies again after one."""
     t = [buffers[n] for n in ("qweight", "g_idx", "scales", "qzeros")]
     v = [None if x.is_inference() else x._version for x in t]
     return (t[0], v[0], t[1], v[1], t[2], v[2], t[3], v[3], None in v)
@@ -134,7 +135,8 @@ class GPTQLinear(torch.nn.Module):
 
     @torch.no_grad()
     def post_init(self) -> "GPTQLinear":
-        """Build the kernel-side weight: for act-order, the group-sorted copy and gather index."""
+        """Build the kernel-side weight: for act-order, the group-sorted copy and gather index;
+        the copies that are there already are made again."""
         if not self._strip_only:
             self._remake(None)
         return self

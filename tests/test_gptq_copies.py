@@ -109,6 +109,18 @@ def test_buffers_changed_after_use(kernels, act):
     assert set(kernels) == {"gemv", "rows", "prompt"}
 
 
+def test_post_init_makes_every_copy_again(kernels):
+    # after a write that torch does not count, here through .data
+    for act in (False, True):
+        lin, other = _linear(1, act), _linear(2, act)
+        for m in ROWS:
+            lin(_x(m))
+        for a, b in zip(lin.buffers(), other.buffers()):
+            a.data.copy_(b)
+        lin.post_init()
+        assert all(torch.equal(lin(_x(m)), other(_x(m))) for m in ROWS)
+
+
 def test_copies_are_made_again_in_place(kernels):
     # a captured graph or a decoder that holds a copy's address reads the new weight through it
     lin = _linear(1, True)
